@@ -1,0 +1,63 @@
+"""The VQ4P int8-table kernels where their tiles end: widths that leave a
+partial group of 4 positions, a partial block of 32 and a partial row block,
+tables of several LDS passes, jobs of 1 to 8 tokens, and launches with one
+and with four row blocks per block. A matvec is bit for bit the oracle's
+(integer sums and a fixed order of fp32 folds); layers meet the 1e-4 bar.
+"""
+import numpy as np
+import pytest
+
+import container as ct
+from gpu_util import BALANCED, dev, empty, host, open_ctx, rel_err
+from oracle import pyoracle as po
+
+pytestmark = pytest.mark.gpu
+
+
+def model_of(hidden, inter, experts=6, top_k=3):
+    return ct.build(ct.Spec(hidden=hidden, inter=inter, experts=experts, top_k=top_k, layers=1, fmt="VQ4P",
+                            shared_bits=0, seed=hidden + inter, keep_codes=False, **BALANCED))
+
+
+@pytest.mark.parametrize("hidden,inter", [(8, 8), (264, 72), (328, 200), (2080, 136), (4104, 64)])
+def test_matvec_bits(hidden, inter):
+    import warp_amd
+    model = model_of(hidden, inter)
+    ctx = open_ctx(model)
+    try:
+        warp_amd.load_container_model(ctx, model)
+        bT = po.books_T(model.books_raw)
+        rng = np.random.default_rng(hidden)
+        for e in (0, 5):
+            raw = model.layers[0].records[e]
+            r, hdr = np.frombuffer(raw, np.uint8), np.frombuffer(raw[:48], np.uint32)
+            for kind in range(3):
+                M, N = (inter, hidden) if kind < 2 else (hidden, inter)
+                x, y = rng.normal(size=N).astype(np.float32), empty(M)
+                ctx.vq_matvec(0, kind, ctx.resident(0, e), dev(x), y)
+                at = int(hdr[8]) + 2 * (0, inter, 2 * inter)[kind]
+                scale = r[at:at + 2 * M].view(np.uint16).copy()
+                ref = po.vq_matvec("VQ4P", r[int(hdr[5 + kind]):].copy(), scale, x, bT, kind * 4, M, N)
+                assert np.array_equal(host(y), ref), (e, kind)
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("hidden,inter,experts,T", [(328, 200, 6, 1), (328, 200, 6, 5), (328, 200, 6, 23),
+                                                    (264, 520, 40, 150), (2080, 136, 6, 37)])
+def test_chunk_jobs(hidden, inter, experts, T):
+    """T = 150 over 40 experts: 450 pairs on 2 x 9 row blocks take the launch
+    with four row blocks per block; the others the one with one."""
+    import warp_amd
+    model = model_of(hidden, inter, experts)
+    ctx = open_ctx(model, max_tokens=T)
+    try:
+        warp_amd.load_container_model(ctx, model)
+        X = np.random.default_rng(T).normal(size=(T, hidden)).astype(np.float32)
+        out = empty((T, hidden))
+        ctx.moe_chunk(0, dev(X), out, T)
+        ctx.sync()
+        ref = po.LayerView(model, 0).moe_chunk(X)[0]
+        assert rel_err(host(out), ref) <= 1e-4
+    finally:
+        ctx.close()

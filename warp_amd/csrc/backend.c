@@ -360,7 +360,7 @@ struct warp_hip_ctx {
     float *xscale;
     float *yg, *yu, *yd;
     uint16_t *xsh;
-    float *xscaleh, *hbuf;
+    float *xscaleh;
     uint16_t *xsp;                /* prefill_fp16: x per pair slot, position-group-major */
     float *xscalep;
     float *shg, *shu, *shh, *sho;
@@ -499,7 +499,6 @@ static int ctx_alloc(warp_hip_ctx *c)
     DMALLOC(c, c->yd, P * He * 4);
     DMALLOC(c, c->xsh, P * I * 2 * 2);
     DMALLOC(c, c->xscaleh, P * 4);
-    DMALLOC(c, c->hbuf, P * I * 4);
     if (prefill_fp16(c)) {
         DMALLOC(c, c->xsp, P * He * 2);
         DMALLOC(c, c->xscalep, P * 4);
@@ -703,7 +702,7 @@ void warp_hip_close(warp_hip_ctx *c)
     free(c->L);
     void *d[] = { c->logits, c->idx, c->w, c->jobs, c->njobs, c->missing, c->xs, c->xscale, c->xsp, c->xscalep,
                   c->yg, c->yu,
-                  c->yd, c->xsh, c->xscaleh, c->hbuf, c->shg, c->shu, c->shh, c->sho, c->lut8, c->lut8d,
+                  c->yd, c->xsh, c->xscaleh, c->shg, c->shu, c->shh, c->sho, c->lut8, c->lut8d,
                   c->lscale, c->lscaled, c->counts, c->offsets, c->pair_tok, c->pair_exp, c->pair_w, c->tok_slots, c->runs,
                   c->xin, c->xout, c->la_logits, c->la_idx, c->la_w, c->table_dev, c->pool, c->part,
                   c->shxs, c->shxscale, c->shxin, c->shxinscale, c->tq_dev, c->crc_tmp, c->crc_bad, c->crc_err, c->xlat, c->ylat, c->yup,
@@ -1866,9 +1865,8 @@ int warp_hip_moe_decode(warp_hip_ctx *c, int layer, const float *x_dev, float *o
     if (use_lut) {
         /* the table kernel reads x in f32 */
     } else if (c->P6) {
-        const size_t nvH = (size_t)He / 8, nblkH = (nvH + WARP_LUT_BLK - 1) / WARP_LUT_BLK;
-        KRN(c, wk_lut_p6(xe, 1, He, books_kind(c, L, 0), c->lut8, c->lscale, c->st));
-        KRN(c, wk_lut_p6(xe, 1, He, books_kind(c, L, 1), c->lut8 + nvH * 256, c->lscale + nblkH, c->st));
+        KRN(c, wk_lut_p6(xe, NULL, 1, He, books_kind(c, L, 0), books_kind(c, L, 1), 0, 0.0f, 0.0f, c->lut8, c->lscale,
+                         c->st));
     } else {
         KRN(c, wk_split(xe, 1, He, c->xs, c->xscale, c->st));
     }
@@ -1955,9 +1953,8 @@ int warp_hip_moe_decode(warp_hip_ctx *c, int layer, const float *x_dev, float *o
         if ((rc = books_of(c, layer, c->h_idx, K, &B))) return rc;
         if (B != L && c->P6 && !use_lut) {
             /* the gate/up tables again, from the selection's codebooks */
-            const size_t nvH = (size_t)He / 8, nblkH = (nvH + WARP_LUT_BLK - 1) / WARP_LUT_BLK;
-            KRN(c, wk_lut_p6(xe, 1, He, books_kind(c, B, 0), c->lut8, c->lscale, c->st));
-            KRN(c, wk_lut_p6(xe, 1, He, books_kind(c, B, 1), c->lut8 + nvH * 256, c->lscale + nblkH, c->st));
+            KRN(c, wk_lut_p6(xe, NULL, 1, He, books_kind(c, B, 0), books_kind(c, B, 1), 0, 0.0f, 0.0f, c->lut8,
+                             c->lscale, c->st));
         }
         KRN(c, wait_copies(c));
         /* (the selection again, now with the job lists: the same picks) */
@@ -2020,12 +2017,10 @@ int warp_hip_moe_decode(warp_hip_ctx *c, int layer, const float *x_dev, float *o
         d_off = gu_floats;
         if ((rc = timing_end(c))) return rc;
     } else if (c->P6) {
-        const size_t nvH = (size_t)He / 8, nblkH = (nvH + WARP_LUT_BLK - 1) / WARP_LUT_BLK;
-        KRN(c, wk_apply_p6(c->jobs, c->njobs, K, 0, c->lut8, c->lscale, c->yg, I, He, c->st));
-        KRN(c, wk_apply_p6(c->jobs, c->njobs, K, 1, c->lut8 + nvH * 256, c->lscale + nblkH, c->yu, I, He, c->st));
-        KRN(c, wk_act(c->yg, c->yu, K, I, g->act_situ, g->situ_beta, g->situ_linear_beta, c->hbuf, c->st));
-        KRN(c, wk_lut_p6(c->hbuf, K, I, books_kind(c, B, 2), c->lut8d, c->lscaled, c->st));
-        KRN(c, wk_apply_p6(c->jobs, c->njobs, K, 2, c->lut8d, c->lscaled, c->yd, He, I, c->st));
+        KRN(c, wk_apply_p6(c->jobs, c->njobs, K, 0, 2, K, c->lut8, c->lscale, 1, yk, I, He, c->n_cu, c->st));
+        KRN(c, wk_lut_p6(c->yg, c->yu, K, I, books_kind(c, B, 2), NULL, g->act_situ, g->situ_beta,
+                         g->situ_linear_beta, c->lut8d, c->lscaled, c->st));
+        KRN(c, wk_apply_p6(c->jobs, c->njobs, K, 2, 1, K, c->lut8d, c->lscaled, K, yk + 2, He, I, c->n_cu, c->st));
     } else {
         if ((rc = timing_begin(c, 0))) return rc;
         KRN(c, wk_vq_matvec(g->fmt, c->jobs, c->njobs, K, 0, 2, B->books, c->xs, c->xscale, yk, I, He, 1, c->st));
@@ -2114,14 +2109,12 @@ int warp_hip_expert_ffn(warp_hip_ctx *c, int layer, int expert, const float *x_d
     }
     float *yk[3] = { c->yg, c->yu, out_dev };
     if (c->P6) {
-        const size_t nvH = (size_t)H / 8, nblkH = (nvH + WARP_LUT_BLK - 1) / WARP_LUT_BLK;
-        KRN(c, wk_lut_p6(x_dev, 1, H, books_kind(c, B, 0), c->lut8, c->lscale, c->st));
-        KRN(c, wk_lut_p6(x_dev, 1, H, books_kind(c, B, 1), c->lut8 + nvH * 256, c->lscale + nblkH, c->st));
-        KRN(c, wk_apply_p6(c->jobs, c->njobs, 1, 0, c->lut8, c->lscale, c->yg, I, H, c->st));
-        KRN(c, wk_apply_p6(c->jobs, c->njobs, 1, 1, c->lut8 + nvH * 256, c->lscale + nblkH, c->yu, I, H, c->st));
-        KRN(c, wk_act(c->yg, c->yu, 1, I, g->act_situ, g->situ_beta, g->situ_linear_beta, c->hbuf, c->st));
-        KRN(c, wk_lut_p6(c->hbuf, 1, I, books_kind(c, B, 2), c->lut8d, c->lscaled, c->st));
-        KRN(c, wk_apply_p6(c->jobs, c->njobs, 1, 2, c->lut8d, c->lscaled, out_dev, H, I, c->st));
+        KRN(c, wk_lut_p6(x_dev, NULL, 1, H, books_kind(c, B, 0), books_kind(c, B, 1), 0, 0.0f, 0.0f, c->lut8,
+                         c->lscale, c->st));
+        KRN(c, wk_apply_p6(c->jobs, c->njobs, 1, 0, 2, 1, c->lut8, c->lscale, 1, yk, I, H, c->n_cu, c->st));
+        KRN(c, wk_lut_p6(c->yg, c->yu, 1, I, books_kind(c, B, 2), NULL, g->act_situ, g->situ_beta,
+                         g->situ_linear_beta, c->lut8d, c->lscaled, c->st));
+        KRN(c, wk_apply_p6(c->jobs, c->njobs, 1, 2, 1, 1, c->lut8d, c->lscaled, 1, yk + 2, H, I, c->n_cu, c->st));
         return 0;
     }
     KRN(c, wk_split(x_dev, 1, H, c->xs, c->xscale, c->st));
@@ -2160,19 +2153,15 @@ static int chunk_experts(warp_hip_ctx *c, int layer, const layer_t *B, const flo
     DEV(c, hipEventRecord(c->ev_before, c->st));
     float *yk[3] = { c->yg, c->yu, c->yd };
     if (c->P6) {
-        const size_t nvH = (size_t)H / 8, nblkH = (nvH + WARP_LUT_BLK - 1) / WARP_LUT_BLK;
-        if (first) {
-            /* per token: gate LUT at [t][0], up LUT at [t][1] */
-            KRN(c, wk_lut_p6(X_dev, T, H, books_kind(c, B, 0), c->lut8, c->lscale, c->st));
-            KRN(c, wk_lut_p6(X_dev, T, H, books_kind(c, B, 1), c->lut8 + (size_t)T * nvH * 256,
-                             c->lscale + (size_t)T * nblkH, c->st));
-        }
-        KRN(c, wk_apply_p6(c->jobs, c->njobs, c->max_jobs, 0, c->lut8, c->lscale, c->yg, I, H, c->st));
-        KRN(c, wk_apply_p6(c->jobs, c->njobs, c->max_jobs, 1, c->lut8 + (size_t)T * nvH * 256,
-                           c->lscale + (size_t)T * nblkH, c->yu, I, H, c->st));
-        KRN(c, wk_act(c->yg, c->yu, P, I, g->act_situ, g->situ_beta, g->situ_linear_beta, c->hbuf, c->st));
-        KRN(c, wk_lut_p6(c->hbuf, P, I, books_kind(c, B, 2), c->lut8d, c->lscaled, c->st));
-        KRN(c, wk_apply_p6(c->jobs, c->njobs, c->max_jobs, 2, c->lut8d, c->lscaled, c->yd, H, I, c->st));
+        /* per token: all gate LUTs, then all up LUTs */
+        if (first)
+            KRN(c, wk_lut_p6(X_dev, NULL, T, H, books_kind(c, B, 0), books_kind(c, B, 1), 0, 0.0f, 0.0f, c->lut8,
+                             c->lscale, c->st));
+        KRN(c, wk_apply_p6(c->jobs, c->njobs, c->max_jobs, 0, 2, P, c->lut8, c->lscale, T, yk, I, H, c->n_cu, c->st));
+        KRN(c, wk_lut_p6(c->yg, c->yu, P, I, books_kind(c, B, 2), NULL, g->act_situ, g->situ_beta,
+                         g->situ_linear_beta, c->lut8d, c->lscaled, c->st));
+        KRN(c, wk_apply_p6(c->jobs, c->njobs, c->max_jobs, 2, 1, P, c->lut8d, c->lscaled, P, yk + 2, H, I, c->n_cu,
+                           c->st));
     } else {
         /* by runs: each expert's records decoded once per WARP_RUN_J jobs */
         if (prefill_fp16(c)) {
@@ -2400,8 +2389,8 @@ int warp_hip_vq_matvec(warp_hip_ctx *c, int layer, int kind, const uint8_t *rec_
     if (c->P6) {
         int8_t *lut = kind == 2 ? c->lut8d : c->lut8;
         float *ls = kind == 2 ? c->lscaled : c->lscale;
-        KRN(c, wk_lut_p6(x_dev, 1, N, books_kind(c, B, kind), lut, ls, c->st));
-        KRN(c, wk_apply_p6(c->jobs, c->njobs, 1, kind, lut, ls, y_dev, M, N, c->st));
+        KRN(c, wk_lut_p6(x_dev, NULL, 1, N, books_kind(c, B, kind), NULL, 0, 0.0f, 0.0f, lut, ls, c->st));
+        KRN(c, wk_apply_p6(c->jobs, c->njobs, 1, kind, 1, 1, lut, ls, 1, &y_dev, M, N, c->n_cu, c->st));
     } else if (use_gather(c, B, 1) && N % 32 == 0) {
         /* one launch of the row kernel: the whole matvec */
         float *yk[3] = { y_dev, y_dev, y_dev };

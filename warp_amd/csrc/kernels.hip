@@ -4971,87 +4971,254 @@ extern "C" int wk_combine(const float *y, const float *w, int K, int H, const fl
 
 // ---- VQ4P: int8 LUT and its apply ------------------------------------------------------------
 
-// One block per (vector, 32-position block): the fp32 LUT entries with the
-// fused d-ascending chain of the reference's AVX-512 build
+// Where entry (stage s, code c) of position v sits in the position's 256
+// bytes: the stages rotate with the position, so that four neighbouring
+// positions' tables of one stage lie on different LDS banks and a wave that
+// looks up four positions at once has no bank conflict (within one table
+// the lanes that share a bank share its word).
+__device__ __forceinline__ int p6_slot(int v, int s) { return ((s + v) & 3) << 6; }
+
+// One block per (vector, 32-position block, codebook set): the fp32 LUT
+// entries with the fused d-ascending chain of the reference's AVX-512 build
 // (src/simd_avx512.c:90-123), then max|.|, scale = max/127, ties-to-even
-// rounding and the +-127 clamp (src/model.c:2048-2109).
-__global__ __launch_bounds__(256) void k_lut_p6(const float *__restrict__ x, int N,
-                                                const uint16_t *__restrict__ books, int8_t *__restrict__ lut8,
-                                                float *__restrict__ lscale) {
-    __shared__ float lut[WARP_LUT_BLK * 256];
+// rounding and the +-127 clamp (src/model.c:2048-2109). ACT: the vector is
+// act(x, u) (the SwiGLU of the gate and up rows). A thread holds one
+// entry's codebook vector and makes it for 8 of the positions; the bytes
+// leave through LDS as 16-byte stores. Set z's tables follow set z - 1's of
+// all vectors. What bounds it is latency: 256 threads with 32 entries each,
+// their codebook values loaded one by one, took 10.6 us for a vector of 288
+// positions, 1024 threads 5.1 us for both the gate and up sets.
+template <bool ACT>
+__global__ __launch_bounds__(1024) void k_lut_p6(const float *__restrict__ x, const float *__restrict__ u, int N,
+                                                 const uint16_t *__restrict__ books0,
+                                                 const uint16_t *__restrict__ books1, int situ, float beta,
+                                                 float lbeta, int8_t *__restrict__ lut8,
+                                                 float *__restrict__ lscale) {
     __shared__ float xsh[WARP_LUT_BLK * 8];
-    const int vec = blockIdx.y, blk = blockIdx.x, nv = N >> 3;
-    const int v0 = blk * WARP_LUT_BLK, v1 = min(v0 + WARP_LUT_BLK, nv), nvb = v1 - v0;
-    const float *xv = x + (size_t)vec * N;
-    for (int i = threadIdx.x; i < nvb * 8; i += blockDim.x) xsh[i] = xv[v0 * 8 + i];
+    __shared__ int8_t out[WARP_LUT_BLK * 256];
+    const int vec = blockIdx.y, blk = blockIdx.x, nv = N >> 3, nblk = (nv + WARP_LUT_BLK - 1) / WARP_LUT_BLK;
+    const int tid = threadIdx.x, e = tid & 255, g = tid >> 8;
+    const int v0 = blk * WARP_LUT_BLK, nvb = min(WARP_LUT_BLK, nv - v0);
+    // the entry's codebook vector, flushed as the loader does
+    const uint4 raw = *(const uint4 *)((blockIdx.z ? books1 : books0) + (size_t)e * 8);
+    if (tid < nvb * 8) {
+        const size_t at = (size_t)vec * N + v0 * 8 + tid;
+        xsh[tid] = ACT ? act_pair(x[at], u[at], situ, beta, lbeta) : x[at];
+    }
+    const unsigned rw[4] = { raw.x, raw.y, raw.z, raw.w };
+    float cv[8];
+#pragma unroll
+    for (int d = 0; d < 8; d++) cv[d] = f16_flushed((uint16_t)(rw[d >> 1] >> (16 * (d & 1))));
     __syncthreads();
-    float m = 0.0f;
-    for (int q = threadIdx.x; q < nvb * 256; q += blockDim.x) {
-        const int v = q >> 8, s = (q >> 6) & 3, c = q & 63;
-        float t = 0.0f;
-        for (int d = 0; d < 8; d++)
-            t = __builtin_fmaf(xsh[v * 8 + d], f16_flushed(books[((size_t)s * 64 + c) * 8 + d]), t);
-        lut[q] = t;
-        m = fmaxf(m, fabsf(t));
+    float t[8], m = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const int v = g * 8 + k;
+        t[k] = 0.0f;
+        if (v < nvb) {
+#pragma unroll
+            for (int d = 0; d < 8; d++) t[k] = __builtin_fmaf(xsh[v * 8 + d], cv[d], t[k]);
+            m = fmaxf(m, fabsf(t[k]));
+        }
     }
     m = block_absmax(m);
     const float inv = m > 0.0f ? __fdiv_rn(127.0f, m) : 0.0f;
-    int8_t *dst = lut8 + ((size_t)vec * nv + v0) * 256;
-    for (int q = threadIdx.x; q < nvb * 256; q += blockDim.x) {
-        int t = (int)rintf(__fmul_rn(lut[q], inv));
-        t = t > 127 ? 127 : (t < -127 ? -127 : t);
-        dst[q] = (int8_t)t;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const int v = g * 8 + k;
+        int q = (int)rintf(__fmul_rn(t[k], inv));
+        q = q > 127 ? 127 : (q < -127 ? -127 : q);
+        out[v * 256 + p6_slot(v, e >> 6) + (e & 63)] = (int8_t)q;
     }
-    if (threadIdx.x == 0) lscale[(size_t)vec * ((nv + WARP_LUT_BLK - 1) / WARP_LUT_BLK) + blk] = __fdiv_rn(m, 127.0f);
+    __syncthreads();
+    const size_t row = (size_t)blockIdx.z * gridDim.y + vec;
+    if (tid < nvb * 16) *(uint4 *)(lut8 + (row * nv + v0) * 256 + tid * 16) = *(const uint4 *)(out + tid * 16);
+    if (tid == 0) lscale[row * nblk + blk] = __fdiv_rn(m, 127.0f);
 }
 
-extern "C" int wk_lut_p6(const float *x, int V, int N, const uint16_t *books_kind, int8_t *lut8, float *lscale,
-                         void *stream) {
-    if (V <= 0 || N <= 0 || (N & 7)) return -1;
+extern "C" int wk_lut_p6(const float *x, const float *u, int V, int N, const uint16_t *books0, const uint16_t *books1,
+                         int act_situ, float beta, float lbeta, int8_t *lut8, float *lscale, void *stream) {
+    if (V <= 0 || N <= 0 || (N & 7) || (((uintptr_t)books0 | (uintptr_t)books1 | (uintptr_t)lut8) & 15)) return -1;
     const int nv = N / 8, nblk = (nv + WARP_LUT_BLK - 1) / WARP_LUT_BLK;
-    hipLaunchKernelGGL(k_lut_p6, dim3(nblk, V), dim3(256), 0, (hipStream_t)stream, x, N, books_kind, lut8, lscale);
+    const dim3 grid(nblk, V, books1 ? 2 : 1);
+    if (u)
+        hipLaunchKernelGGL(k_lut_p6<true>, grid, dim3(1024), 0, (hipStream_t)stream, x, u, N, books0, books1,
+                           act_situ, beta, lbeta, lut8, lscale);
+    else
+        hipLaunchKernelGGL(k_lut_p6<false>, grid, dim3(1024), 0, (hipStream_t)stream, x, u, N, books0, books1,
+                           act_situ, beta, lbeta, lut8, lscale);
     CHECK_LAUNCH();
     return 0;
 }
 
-// One wave per (job, 64-row block), lane = row: integer block sums of the
-// four int8 lookups, folded into fp32 once per 32 positions in the
-// reference's order (src/model.c:2136-2229, portable branch).
-__global__ __launch_bounds__(256) void k_apply_p6(const warp_job *__restrict__ jobs, const int *__restrict__ njobs,
-                                                  int kind, const int8_t *__restrict__ lut8,
-                                                  const float *__restrict__ lscale, float *__restrict__ y, int M,
-                                                  int N) {
-    const int nv = N >> 3, nrb = (M + 63) >> 6, nblk = (nv + WARP_LUT_BLK - 1) / WARP_LUT_BLK;
-    const int unit = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (unit >= njobs[kind] * nrb) return;
-    const warp_job &jb = jobs[unit / nrb];
-    const int rb = unit % nrb, r = rb * 64 + lane;
-    const uint8_t *idx = jb.idx;
-    for (int ts = 0; ts < jb.n; ts++) {
-    const int8_t *T0 = lut8 + (size_t)jb.xi[ts] * nv * 256;
-    const float *ls = lscale + (size_t)jb.xi[ts] * nblk;
-    float acc = 0.0f;
-    for (int b = 0; b < nblk; b++) {
-        const int v0 = b * WARP_LUT_BLK, v1 = min(v0 + WARP_LUT_BLK, nv);
-        int sum = 0;
-        for (int v = v0; v < v1; v++) {
-            const uint8_t *p = idx + (((size_t)rb * nv + v) * 64 + lane) * 3;
-            const int8_t *T = T0 + (size_t)v * 256;
-            sum += T[code_at<WARP_FMT_VQ4P>(p, 0)] + T[64 + code_at<WARP_FMT_VQ4P>(p, 1)] +
-                   T[128 + code_at<WARP_FMT_VQ4P>(p, 2)] + T[192 + code_at<WARP_FMT_VQ4P>(p, 3)];
+struct P6Args {
+    const warp_job *jobs;       // the kinds' lists, max_jobs each
+    const int *njobs;
+    int max_jobs, kind_lo;
+    const int8_t *lut8[2];      // per kind: [nx][nv][256]
+    const float *lscale[2];     // [nx][nblk]
+    float *y[2];                // [ny][M]
+    int M, N;
+};
+
+constexpr int P6_NW = 8;        // waves per block
+constexpr int P6_LDS = 65536;   // table bytes per pass
+
+// One job's RB row blocks of 64 against its TK input vectors (of which n
+// are in use). Lane l looks up 4 rows (l & 15) at position 4 k + (l >> 4):
+// a 12-byte code word, 16 addresses, made once for all the vectors.
+template <int TK, int RB>
+__device__ __forceinline__ void p6_rows(const P6Args &a, const warp_job &jb, int n, int kind, int rb0, int8_t *lds,
+                                        int *isum) {
+    constexpr int PS = P6_LDS / 256 / TK / WARP_LUT_BLK * WARP_LUT_BLK;     // positions per pass
+    constexpr int NB = PS / WARP_LUT_BLK;
+    constexpr int GP = PS / 4 * RB / P6_NW;                                 // groups of 4 positions per wave
+    constexpr int CH = GP < 8 ? GP : 8;                                     // of which one 32-position block
+    constexpr int D = GP < 4 ? GP : 4;                                      // code words ahead
+    constexpr int NR = TK * RB * 64, NA = (NR + P6_NW * 64 - 1) / (P6_NW * 64);
+    const int nv = a.N >> 3, nrb = (a.M + 63) >> 6, nblk = (nv + WARP_LUT_BLK - 1) / WARP_LUT_BLK;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4;
+    const int rw = wave % RB, sub = wave / RB, rb = min(rb0 + rw, nrb - 1);
+    const uint8_t *idx = jb.idx + (size_t)rb * nv * 192 + (lane & 15) * 12;
+    int xi[TK];
+#pragma unroll
+    for (int t = 0; t < TK; t++) xi[t] = jb.xi[t < n ? t : 0];
+    float acc[NA];
+#pragma unroll
+    for (int i = 0; i < NA; i++) acc[i] = 0.0f;
+    int base[4];
+#pragma unroll
+    for (int s = 0; s < 4; s++) base[s] = g * 256 + p6_slot(g, s) + sub * GP * 1024;
+    for (int p0 = 0; p0 < nv; p0 += PS) {
+        // the first code words, then the tables (zeros past the end)
+        Word<3> wd[D];
+        const int k0 = p0 / 4 + sub * GP;
+        auto word = [&](int j, int k) {
+            wd[j].load_keep(idx + (size_t)min((k0 + min(k, GP - 1)) * 4 + g, nv - 1) * 192);
+        };
+#pragma unroll
+        for (int j = 0; j < D; j++) word(j, j);
+#pragma unroll
+        for (int t = 0; t < TK; t++) {
+            const int8_t *src = a.lut8[kind] + ((size_t)xi[t] * nv + p0) * 256;
+            const int lim = (nv - p0) * 256;
+#pragma unroll
+            for (int o = 0; o < PS * 256; o += P6_NW * 64 * 16) {
+                const int at = o + tid * 16;
+                uint4 q = make_uint4(0, 0, 0, 0);
+                if (at < lim && at < PS * 256) q = *(const uint4 *)(src + at);
+                if (at < PS * 256) *(uint4 *)(lds + t * PS * 256 + at) = q;
+            }
         }
-        acc = __fadd_rn(acc, __fmul_rn(ls[b], (float)sum));
+        for (int i = tid; i < NB * NR; i += P6_NW * 64) isum[i] = 0;
+        __syncthreads();
+#pragma unroll 1
+        for (int c = 0; c < GP / CH; c++) {
+            int sum[TK][4];
+#pragma unroll
+            for (int t = 0; t < TK; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) sum[t][r] = 0;
+#pragma unroll 1
+            for (int k = c * CH; k < c * CH + CH; k += D) {
+#pragma unroll
+                for (int j = 0; j < D; j++) {
+                    const Word<3> wk = wd[j];
+                    word(j, k + j + D);                    // (its share's last again at the end)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const unsigned w = wk.slot(r);
+                        const int8_t *at[4];
+#pragma unroll
+                        for (int s = 0; s < 4; s++) at[s] = lds + (((w >> (6 * s)) & 63u) + base[s] + k * 1024);
+#pragma unroll
+                        for (int t = 0; t < TK; t++)
+                            sum[t][r] += (at[0][j * 1024 + t * PS * 256] + at[1][j * 1024 + t * PS * 256]) +
+                                         (at[2][j * 1024 + t * PS * 256] + at[3][j * 1024 + t * PS * 256]);
+                        // (the sums kept in this order: reassociated over the
+                        // steps, their terms would not fit the registers)
+#pragma unroll
+                        for (int t = 0; t < TK; t++) asm volatile("" : "+v"(sum[t][r]));
+                    }
+                }
+            }
+            // over the wave's four positions: lane group g ends with row
+            // 4 (l & 15) + g
+            const int b = (sub * GP + c * CH) >> 3;
+#pragma unroll
+            for (int t = 0; t < TK; t++) {
+                const auto h0 = __builtin_amdgcn_permlane32_swap(sum[t][0], sum[t][2], false, false);
+                const auto h1 = __builtin_amdgcn_permlane32_swap(sum[t][1], sum[t][3], false, false);
+                const int s0 = (int)(h0[0] + h0[1]), s1 = (int)(h1[0] + h1[1]);   // rows 0, 1 below; 2, 3 above
+                const auto q = __builtin_amdgcn_permlane16_swap(s0, s1, false, false);
+                atomicAdd(isum + ((b * TK + t) * RB + rw) * 64 + (lane & 15) * 4 + g, (int)(q[0] + q[1]));
+            }
+        }
+        __syncthreads();
+        // folded once per 32 positions in the reference's order
+#pragma unroll
+        for (int i = 0; i < NA; i++) {
+            const int at = tid + i * P6_NW * 64, t = at / (RB * 64);
+            if (at < NR) {
+                const float *ls = a.lscale[kind] + (size_t)jb.xi[t < n ? t : 0] * nblk + p0 / WARP_LUT_BLK;
+                for (int b = 0; b < NB && p0 / WARP_LUT_BLK + b < nblk; b++)
+                    acc[i] = __fadd_rn(acc[i], __fmul_rn(ls[b], (float)isum[b * NR + at]));
+            }
+        }
+        __syncthreads();
     }
-    if (r < M) y[(size_t)jb.yi[ts] * M + r] = __fmul_rn(acc, f16_keep(jb.scale[r]));
+#pragma unroll
+    for (int i = 0; i < NA; i++) {
+        const int at = tid + i * P6_NW * 64, t = at / (RB * 64), r = rb0 * 64 + at % (RB * 64);
+        if (at < NR && t < n && r < a.M)
+            a.y[kind][(size_t)jb.yi[t] * a.M + r] = __fmul_rn(acc[i], f16_keep(jb.scale[r]));
     }
 }
 
-extern "C" int wk_apply_p6(const warp_job *jobs, const int *njobs, int max_jobs, int kind, const int8_t *lut8,
-                           const float *lscale, float *y, int M, int N, void *stream) {
-    if (M <= 0 || N <= 0 || (N & 7) || kind < 0 || kind > 2 || max_jobs <= 0) return -1;
-    const int nrb = (M + 63) / 64, units = max_jobs * nrb;
-    hipLaunchKernelGGL(k_apply_p6, dim3((units + 3) / 4), dim3(256), 0, (hipStream_t)stream,
-                       jobs + (size_t)kind * max_jobs, njobs, kind, lut8, lscale, y, M, N);
+// A block per (kind, job, RB row blocks): integer block sums of the four
+// int8 lookups per position, folded into fp32 once per 32 positions in the
+// reference's order (src/model.c:2136-2229, portable branch), so the split of
+// the positions over the block's waves changes no bit. The tables of the
+// job's input vectors are staged in LDS a pass at a time (64 KiB: two blocks
+// per CU), where a lookup is one ds_read of a byte without conflicts (the
+// rotation of p6_slot); looked up in global memory, one wave per row block
+// and one vector at a time, the apply of one decode layer (8 experts of
+// 2304 x 1024) took 437 us in three launches and takes 22 us in two now.
+template <int RB>
+__global__ __launch_bounds__(P6_NW * 64) void k_apply_p6(P6Args a) {
+    __shared__ __attribute__((aligned(16))) int8_t lds[P6_LDS];
+    __shared__ int isum[P6_LDS / 256 / WARP_LUT_BLK * RB * 64];
+    const int kind = blockIdx.y, nrg = (((a.M + 63) >> 6) + RB - 1) / RB;
+    const int job = blockIdx.x / nrg, rb0 = (blockIdx.x % nrg) * RB;
+    if (job >= a.njobs[a.kind_lo + kind]) return;
+    const warp_job &jb = a.jobs[(size_t)(a.kind_lo + kind) * a.max_jobs + job];
+    const int n = jb.n;
+    if (n <= 1) p6_rows<1, RB>(a, jb, n, kind, rb0, lds, isum);
+    else if (n == 2) p6_rows<2, RB>(a, jb, n, kind, rb0, lds, isum);
+    else if (n <= 4) p6_rows<4, RB>(a, jb, n, kind, rb0, lds, isum);
+    else p6_rows<8, RB>(a, jb, n, kind, rb0, lds, isum);
+}
+
+extern "C" int wk_apply_p6(const warp_job *jobs, const int *njobs, int max_jobs, int kind_lo, int nkinds, int pairs,
+                           const int8_t *lut8, const float *lscale, int nvec, float *const *y, int M, int N, int n_cu,
+                           void *stream) {
+    if (M <= 0 || N <= 0 || (N & 7) || kind_lo < 0 || nkinds < 1 || nkinds > 2 || kind_lo + nkinds > 3 ||
+        max_jobs <= 0 || ((uintptr_t)lut8 & 15))
+        return -1;
+    const int nv = N / 8, nblk = (nv + WARP_LUT_BLK - 1) / WARP_LUT_BLK, nrb = (M + 63) / 64;
+    P6Args a = { jobs, njobs, max_jobs, kind_lo, { lut8, lut8 + (size_t)nvec * nv * 256 },
+                 { lscale, lscale + (size_t)nvec * nblk }, { y[0], nkinds > 1 ? y[1] : y[0] }, M, N };
+    // Four row blocks per block share its staged tables once that leaves
+    // two blocks for every CU (pairs bounds the jobs there are): a layer's
+    // 192 pairs of 24 tokens take 249 us with four, 258 with two and 294
+    // with one, which a decode's few jobs need to fill the chip.
+    const long jobs_most = pairs < max_jobs ? pairs : max_jobs;
+    if (jobs_most * nkinds * nrb >= 8L * n_cu)
+        hipLaunchKernelGGL(k_apply_p6<4>, dim3((unsigned)(max_jobs * ((nrb + 3) / 4)), nkinds), dim3(P6_NW * 64), 0,
+                           (hipStream_t)stream, a);
+    else
+        hipLaunchKernelGGL(k_apply_p6<1>, dim3((unsigned)(max_jobs * nrb), nkinds), dim3(P6_NW * 64), 0,
+                           (hipStream_t)stream, a);
     CHECK_LAUNCH();
     return 0;
 }

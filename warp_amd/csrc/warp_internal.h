@@ -316,14 +316,20 @@ int wk_act_split(const float *g, const float *u, int P, int I, int act_situ,
 int wk_combine(const float *y, const float *w, int K, int H, const float *add0,
                const float *add1, const int *missing, float *out, void *stream);
 
-/* VQ4P: int8 LUT of x for one kind (4 stages x 64 entries, one scale per 32
+/* VQ4P: int8 LUT of x, or of act(x, u) where u is given, for one codebook
+ * set or two (books1 not NULL; 4 stages x 64 entries, one scale per 32
  * positions), bit-identical to the reference's fused LUT build and
- * quantisation. x [V][N] f32 -> lut8 [V][N/8][4][64], lscale [V][nblk]. */
-int wk_lut_p6(const float *x, int V, int N, const uint16_t *books_kind, int8_t *lut8,
-              float *lscale, void *stream);
-/* VQ4P apply over a job list of one kind: y[yi] = apply(rec kind, lut8[xi]). */
-int wk_apply_p6(const warp_job *jobs, const int *njobs, int max_jobs, int kind,
-                const int8_t *lut8, const float *lscale, float *y, int M, int N,
+ * quantisation. x, u [V][N] f32 -> lut8 [sets][V][N/8][256], the stages of a
+ * position in an order of wk_apply_p6's own, lscale [sets][V][nblk]. Books
+ * and lut8 16-byte aligned. */
+int wk_lut_p6(const float *x, const float *u, int V, int N, const uint16_t *books0, const uint16_t *books1,
+              int act_situ, float beta, float lbeta, int8_t *lut8, float *lscale, void *stream);
+/* VQ4P apply over the job lists of kinds kind_lo .. kind_lo + nkinds - 1 (1
+ * or 2; max_jobs apart in jobs): y[k][yi] = apply(rec kind, lut8[k][xi]),
+ * lut8 and lscale as wk_lut_p6 leaves them for nvec vectors. pairs: the
+ * most (input, record) pairs a list holds. */
+int wk_apply_p6(const warp_job *jobs, const int *njobs, int max_jobs, int kind_lo, int nkinds, int pairs,
+                const int8_t *lut8, const float *lscale, int nvec, float *const *y, int M, int N, int n_cu,
                 void *stream);
 /* silu/SiTU pairs for VQ4P: h [P][I] = act(g, u), exactly as the reference. */
 int wk_act(const float *g, const float *u, int P, int I, int act_situ, float beta,
