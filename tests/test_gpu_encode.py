@@ -84,3 +84,41 @@ def test_lloyd_matches_reference():
         assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), it
         C0 = ref
     log(f"vq_lloyd: 3 iterations over {n} vectors, {E} clusters (56 empty) bit-identical to waste_vq_lloyd")
+
+
+@pytest.mark.parametrize("S,E,n", [
+    (1, 1, 1), (2, 15, 63), (3, 16, 65), (3, 17, 1000), (17, 16, 130), (3, 255, 20001), (3, 256, 131072 + 1),
+    (4, 257, 3000), (3, 512, 3000), (2, 1024, 3000), (2, 1025, 3000), (1, 2000, 131072 - 63), (2, 4095, 3000)])
+def test_encode_scores_never_decide(S, E, n):
+    """The winner the matrix cores propose is confirmed or the vector scanned:
+    codes equal the oracle's at the edges of tiles (16 entries), of their
+    numbering (256), of LDS pieces (1024), of launches (96 tiles, 16 stages)
+    and of blocks, for duplicated entries in one group of 4 and across groups,
+    vectors on entries and on zero, vectors and codebooks out of the scores'
+    range, infinities and NaN."""
+    import warp_amd.hip as wh
+    rng = np.random.default_rng(1000 * S + E)
+    books = (rng.normal(0.0, 1.0, size=(S, E, 8)) * 0.6 ** np.arange(S)[:, None, None]).astype(np.float32)
+    X = rng.normal(0.0, 1.0, size=(n, 8)).astype(np.float32)
+    for i in range(1, 40):                            # duplicates, near and far
+        books[rng.integers(S), rng.integers(E)] = books[rng.integers(S), rng.integers(E)]
+    books[0, E // 2] = 0.0
+    m = min(n, 40)
+    X[:m] = books[0, rng.integers(0, E, m)]
+    X[m // 2:m] = 0.0
+    for i, v in enumerate([np.nan, np.inf, -np.inf, 3e38, 1e25, 1e10, 1e-30, 1e-42, 100.0]):
+        X[(7 + 61 * i) % n, i % 8] = v                # one component
+        with np.errstate(over="ignore", invalid="ignore"):
+            X[(11 + 67 * i) % n] *= np.float32(v)
+    kinds = {"": books}
+    if n <= 3000:
+        with np.errstate(over="ignore"):
+            kinds.update(offset=books + np.float32(300.0), tiny=books * np.float32(1e-25), huge=books * np.float32(1e25),
+                         zero=books * 0.0)
+        kinds["bad"] = books.copy()
+        kinds["bad"][0, E // 3, 3], kinds["bad"][S - 1, E // 4, 0] = np.nan, np.inf
+    for kind, b in kinds.items():
+        b = np.ascontiguousarray(b, dtype=np.float32)
+        got, ref = wh.vq_encode(X, b), np.empty((n, S), np.uint16)
+        po.lib().or_vq_encode(X.ctypes.data, n, b.ctypes.data, S, E, 8, ref.ctypes.data)
+        assert np.array_equal(got, ref), (kind, int(np.count_nonzero(got != ref)))

@@ -5597,47 +5597,309 @@ extern "C" int wk_combine_chunk(const float *y, const int *tok_slots, const floa
 // nearest the current vector under squared L2, d = sum over j ascending of
 // (v[j] - e[j])^2 with every multiply and add rounded on its own (the
 // reference's vq.c is built without FMA), the first minimum winning
-// (strict <), then the exact residual v - e feeds the next stage. One launch
-// per stage: the stage's codebook (entries x 8 fp32, up to 128 KiB) in LDS,
-// one thread per vector scanning every entry (all lanes read the same entry
-// at once: LDS broadcasts). The residual is kept in `cur`. Blocks of 1024
-// threads, so that a 4096-entry codebook (128 KiB, one block per CU) still
-// leaves 4 waves per SIMD.
-constexpr int ENC_NT = 1024;
+// (strict <), then the exact residual v - e feeds the next stage.
+//
+// Taken literally that is 27 vector instructions per vector and entry, and
+// the scan was bound by them. Here the matrix cores find the winner and the
+// reference's arithmetic only confirms it. d / 2 orders entries as the score
+// |e|^2 / 2 - v . e + B does (B of the vector alone, about |v|^2 / 2), and one
+// v_mfma_f32_16x16x32_f16 gives 16 entries x 16 vectors of that: v and e,
+// scaled by a power of two that puts the codebook's largest component into
+// [512, 1024), are split into fp16 high and low parts, and the 32 products of
+// a pair are
+//   k  0.. 7  -v high . e high      k 24..26  256 . (|e|^2 / 512 in three parts)
+//   k  8..15  -v high . e low       k 27      2^15 . (0, or past the codebook's
+//   k 16..23  -v low . e high                 end a value no score reaches)
+//                                   k 28      B / 2^14 . 2^14
+// Scores are positive (B has a margin), so they compare as whole numbers. A
+// lane holds 4 entries of one vector; their least score, its low four bits
+// replaced by the number of the 16-entry tile, goes into a running least and
+// second least. So a wave has, for its 64 vectors, the best group
+// of 4 entries and a bound on every other group. If the second least is
+// further off than the scores can be wrong (see enc_margin), the reference's
+// winner is in that group, and its 4 entries are compared with the
+// reference's own arithmetic; any other vector (near ties, infinities, NaN,
+// magnitudes out of range) is scanned in full by the whole wave. Codes are
+// those of the scan in every case.
+//
+// Bound by the vector instructions of the running minimum and the matrix
+// cores about alike. Stages whose codebooks fit LDS together go in one
+// launch, the residual in registers: 1,835,008 vectors, 3 x 256 entries,
+// 154 us (the scan: 698). A larger codebook goes one stage a launch, 1,024
+// entries staged at a time: the same vectors against 2 x 4,096, 1,519 us (the
+// scan: 7,674).
+constexpr int ENC_TILES = 96;                        // 16-entry tiles in LDS at most (1 KiB each), all stages in a launch
+constexpr int ENC_PIECE = 64;                        // tiles staged at a time when a stage's are more
+constexpr int ENC_STAGES = 16;                       // stages in a launch at most
 
-__global__ __launch_bounds__(ENC_NT) void k_vq_encode_stage(const float *__restrict__ X, float *__restrict__ cur,
-                                                            const float *__restrict__ book, int entries, long n,
-                                                            int stage, int stages, uint16_t *__restrict__ codes) {
-    extern __shared__ float4 cb4[];                  // [entries][2] float4
-    for (int i = threadIdx.x; i < entries * 2; i += ENC_NT) cb4[i] = ((const float4 *)book)[i];
-    __syncthreads();
-    const long i = (long)blockIdx.x * ENC_NT + threadIdx.x;
-    if (i >= n) return;
-    const float4 *src = (const float4 *)((stage == 0 ? X : cur) + i * 8);
-    const float4 v0 = src[0], v1 = src[1];
-    const float v[8] = { v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w };
-    int best = 0;
-    float bestd = INFINITY;
-    for (int c = 0; c < entries; c++) {
-        const float4 e0 = cb4[2 * c], e1 = cb4[2 * c + 1];
-        const float e[8] = { e0.x, e0.y, e0.z, e0.w, e1.x, e1.y, e1.z, e1.w };
-        float d = 0.0f;
+struct EncArgs {
+    const float *src;                                // [n][8]
+    float *dst;                                      // the residual for the next launch's stages, or null
+    const float *books;                              // the launch's stages [nst][entries][8]
+    long n;
+    int entries, nst, stage0, stages;
+    uint16_t *codes;                                 // [n][stages]
+};
+
+// How far below the least score of the other groups the winner's must be.
+// With V = |v|, E = max |e| (both scaled), the products of a score sum to at
+// most 1.01 (V + E)^2 / 2 + 2^15 in magnitude. A score's error is at most
+// 2^-17 of that (32 products added in fp32 in any order, truncated at worst:
+// 2^-18; the tile number in the four low bits: 2^-19; the products of the
+// splits' remainders: 2^-20) plus 2^-12 (V + E + 64) where parts fall below
+// the normal fp16 range; the reference's d / 2 is rounded by at most
+// 2^-20 (V + E)^2. Twice their sum, as two scores are compared.
+__device__ __forceinline__ float enc_margin(float V, float E) {
+    const float s = V + E;
+    return 2.02f * (0x1.4p-18f * s * s + 0x1p-12f * (s + 64.0f) + 0.25f);
+}
+
+// the reference's distance
+__device__ __forceinline__ float enc_dist(const float *v, float4 e0, float4 e1) {
+    const float e[8] = { e0.x, e0.y, e0.z, e0.w, e1.x, e1.y, e1.z, e1.w };
+    float d = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const float t = __fsub_rn(v[j], e[j]);
-            d = __fadd_rn(d, __fmul_rn(t, t));
-        }
-        if (d < bestd) {
-            bestd = d;
-            best = c;
-        }
+    for (int j = 0; j < 8; j++) {
+        const float t = __fsub_rn(v[j], e[j]);
+        d = __fadd_rn(d, __fmul_rn(t, t));
     }
-    codes[i * stages + stage] = (uint16_t)best;
-    if (stage + 1 < stages) {
-        const float4 b0 = cb4[2 * best], b1 = cb4[2 * best + 1];
-        float4 *dst = (float4 *)(cur + i * 8);
-        dst[0] = make_float4(__fsub_rn(v[0], b0.x), __fsub_rn(v[1], b0.y), __fsub_rn(v[2], b0.z), __fsub_rn(v[3], b0.w));
-        dst[1] = make_float4(__fsub_rn(v[4], b1.x), __fsub_rn(v[5], b1.y), __fsub_rn(v[6], b1.z), __fsub_rn(v[7], b1.w));
+    return d;
+}
+
+// least and second least score (as bits), and the least's group
+struct EncBest {
+    unsigned k1, k2, id;
+};
+__device__ __forceinline__ EncBest enc_min(const EncBest &x, const EncBest &y) {
+    return { min(x.k1, y.k1), min(max(x.k1, y.k1), min(x.k2, y.k2)), y.k1 < x.k1 ? y.id : x.id };
+}
+// (x, y) -> the halves (SW 32) or the odd and even rows (SW 16) that belong
+// to x's tile in its own lanes and to y's in the others, combined
+template <int SW>
+__device__ __forceinline__ EncBest enc_fold(const EncBest &x, const EncBest &y) {
+    EncBest p, q;
+    auto sw = [](unsigned a, unsigned b, unsigned &ra, unsigned &rb) {
+        const auto r = SW == 32 ? __builtin_amdgcn_permlane32_swap(a, b, false, false)
+                                : __builtin_amdgcn_permlane16_swap(a, b, false, false);
+        ra = r[0];
+        rb = r[1];
+    };
+    sw(x.k1, y.k1, p.k1, q.k1);
+    sw(x.k2, y.k2, p.k2, q.k2);
+    sw(x.id, y.id, p.id, q.id);
+    return enc_min(p, q);
+}
+
+// PIECES: the launch's one stage is staged ENC_PIECE tiles at a time;
+// otherwise every stage's tiles are staged once and a block's waves go over
+// their 64-vector tiles on their own.
+template <bool PIECES>
+__global__ __launch_bounds__(1024) void k_vq_encode(EncArgs a) {
+    extern __shared__ half8 enc_lds[];               // [tiles][64] operands, then [wave][3][64] vector operands
+    __shared__ unsigned s_max[ENC_STAGES], s_norm[ENC_STAGES];   // bits of max |component|, of max |e'|^2
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nt = (a.entries + 15) >> 4;
+    const int nw = blockDim.x >> 6;
+    half8 *xch = enc_lds + (PIECES ? ENC_PIECE : a.nst * nt) * 64 + wave * 192;
+    if (tid < ENC_STAGES) s_max[tid] = s_norm[tid] = 0u;
+    __syncthreads();
+    for (int s = 0; s < a.nst; s++) {
+        const uint4 *b = (const uint4 *)(a.books + (size_t)s * a.entries * 8);
+        unsigned m = 0;
+        for (int i = tid; i < a.entries * 2; i += blockDim.x) {
+            const uint4 w = b[i];
+            m = max(max(m, w.x & 0x7fffffffu), max(w.y & 0x7fffffffu, max(w.z & 0x7fffffffu, w.w & 0x7fffffffu)));
+        }
+        atomicMax(&s_max[s], m);                     // infinities and NaN come out largest
+    }
+    __syncthreads();
+    // 2^x of a stage's scale; a codebook out of range is scanned in full
+    auto scale_of = [&](int s, bool &ok) {
+        const int e = (int)(s_max[s] >> 23) - 126;   // the largest component is in [2^(e - 1), 2^e)
+        ok = e >= -40 && e <= 40;
+        return ok ? ldexpf(1.0f, 10 - e) : 1.0f;
+    };
+    auto stage_tiles = [&](int s, int t0, int t1, half8 *to) {
+        bool ok;
+        const float sc = scale_of(s, ok);
+        const float *b = a.books + (size_t)s * a.entries * 8;
+        float most = 0.0f;
+        for (int c = t0 * 16 + tid; c < t1 * 16; c += blockDim.x) {
+            half8 h = {}, l = {}, k = {};
+            if (c < a.entries) {
+                const float4 e0 = ((const float4 *)b)[2 * c], e1 = ((const float4 *)b)[2 * c + 1];
+                const float e[8] = { e0.x, e0.y, e0.z, e0.w, e1.x, e1.y, e1.z, e1.w };
+                float nn = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const float x = e[j] * sc;
+                    h[j] = (_Float16)x;
+                    l[j] = (_Float16)(x - (float)h[j]);
+                    nn += x * x;
+                }
+                most = fmaxf(most, nn);
+                nn *= 1.0f / 512.0f;
+                k[0] = (_Float16)nn;
+                nn -= (float)k[0];
+                k[1] = (_Float16)nn;
+                nn -= (float)k[1];
+                k[2] = (_Float16)nn;
+            } else {
+                k[3] = (_Float16)60000.0f;
+            }
+            k[4] = (_Float16)16384.0f;
+            half8 *d = to + (size_t)((c >> 4) - t0) * 64 + (c & 15);
+            d[0] = h;
+            d[16] = l;
+            d[32] = h;
+            d[48] = k;
+        }
+        atomicMax(&s_norm[s], __float_as_uint(most));
+    };
+    if (!PIECES) {
+        for (int s = 0; s < a.nst; s++) stage_tiles(s, 0, nt, enc_lds + (size_t)s * nt * 64);
+        __syncthreads();
+    }
+    const int kg = lane >> 4, col = lane & 15;
+    const long ntile = (a.n + 63) >> 6, step = (long)gridDim.x * nw;
+    // (PIECES: one tile per wave, and every wave takes part in the staging)
+    for (long tile = (long)blockIdx.x * nw + wave; PIECES || tile < ntile; tile += step) {
+        const long i = tile * 64 + lane;
+        const bool valid = i < a.n;
+        const float4 *src = (const float4 *)(a.src + (valid ? i : a.n - 1) * 8);
+        const float4 v0 = src[0], v1 = src[1];
+        float v[8] = { v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w };
+        for (int s = 0; s < a.nst; s++) {
+            bool ok;
+            const float sc = scale_of(s, ok);
+            float V2 = 0.0f;
+            half8 h, l;
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const float x = -v[j] * sc;
+                h[j] = (_Float16)x;
+                l[j] = (_Float16)(x - (float)h[j]);
+                V2 += x * x;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            xch[lane] = h;
+            xch[64 + lane] = l;
+            // B: no score is negative, as E < 2900; rounded up (to at least 2)
+            const float V = sqrtf(V2), B = 0.5f * V2 + enc_margin(V, 2900.0f);
+            const half8 konst = { (_Float16)256.0f, (_Float16)256.0f, (_Float16)256.0f, (_Float16)32768.0f,
+                                  (_Float16)(B * 0x1.01p-14f + 0x1p-13f), (_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f };
+            xch[128 + lane] = konst;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            half8 b[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) b[q] = xch[(kg == 3 ? 128 : kg == 2 ? 64 : 0) + q * 16 + col];
+            EncBest r[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) r[q] = { ~0u, ~0u, 0u };
+            // tiles t0 .. t1 - 1 of the stage, 16 (one tile number's worth) at a time
+            auto scan = [&](const half8 *fr, int t0, int t1) {
+                for (int c0 = t0; c0 < t1; c0 += 16, fr += 16 * 64) {
+                    unsigned c1[4], c2[4];
+#pragma unroll
+                    for (int q = 0; q < 4; q++) c1[q] = c2[q] = 0x7f800000u;
+                    auto tile16 = [&](int t) {
+                        const half8 av = fr[t * 64 + lane];
+                        f4 d[4];
+#pragma unroll
+                        for (int q = 0; q < 4; q++)
+                            d[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, b[q], f4{ 0.0f, 0.0f, 0.0f, 0.0f }, 0, 0, 0);
+#pragma unroll
+                        for (int q = 0; q < 4; q++) {
+                            unsigned g = min(min(__float_as_uint(d[q][0]), __float_as_uint(d[q][1])),
+                                             min(__float_as_uint(d[q][2]), __float_as_uint(d[q][3])));
+                            g = (g & ~15u) | (unsigned)t;
+                            // the median: c1 <= c2, all positive
+                            c2[q] = __float_as_uint(__builtin_amdgcn_fmed3f(__uint_as_float(c1[q]), __uint_as_float(c2[q]),
+                                                                            __uint_as_float(g)));
+                            c1[q] = min(c1[q], g);
+                        }
+                    };
+                    const int nc = min(16, t1 - c0);
+                    int t = 0;
+                    for (; t + 4 <= nc; t += 4) {
+                        tile16(t);
+                        tile16(t + 1);
+                        tile16(t + 2);
+                        tile16(t + 3);
+                    }
+                    for (; t < nc; t++) tile16(t);
+#pragma unroll
+                    for (int q = 0; q < 4; q++)
+                        r[q] = enc_min(r[q], { c1[q], c2[q], (unsigned)(c0 * 4) + (c1[q] & 15u) * 4 + kg });
+                }
+            };
+            if (PIECES) {
+                for (int t0 = 0; t0 < nt; t0 += ENC_PIECE) {
+                    const int t1 = min(t0 + ENC_PIECE, nt);
+                    __syncthreads();                 // the piece before is done with
+                    stage_tiles(s, t0, t1, enc_lds);
+                    __syncthreads();
+                    scan(enc_lds, t0, t1);
+                }
+            } else {
+                scan(enc_lds + (size_t)s * nt * 64, 0, nt);
+            }
+            // lane l gets vector l's: tiles 0 and 2, 1 and 3 by halves, then by rows
+            const EncBest w = enc_fold<16>(enc_fold<32>(r[0], r[2]), enc_fold<32>(r[1], r[3]));
+            const float E = sqrtf(__uint_as_float(s_norm[s]));
+            const bool cert = ok && V <= 16384.0f && __uint_as_float(w.k2) - __uint_as_float(w.k1) > enc_margin(V, E);
+            const float4 *bk = (const float4 *)(a.books + (size_t)s * a.entries * 8);
+            int best = 0;
+            float bestd = INFINITY;
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int c = (int)w.id * 4 + u, cc = min(c, a.entries - 1);
+                const float d = enc_dist(v, bk[2 * cc], bk[2 * cc + 1]);
+                if (c < a.entries && d < bestd) {
+                    bestd = d;
+                    best = c;
+                }
+            }
+            for (uint64_t todo = __ballot(valid && !cert); todo; todo &= todo - 1) {
+                const int at = __ffsll((unsigned long long)todo) - 1;
+                float x[8];
+#pragma unroll
+                for (int j = 0; j < 8; j++) x[j] = __shfl(v[j], at);
+                float md = INFINITY;
+                int mc = 0x7fffffff;
+                for (int c = lane; c < a.entries; c += 64) {
+                    const float d = enc_dist(x, bk[2 * c], bk[2 * c + 1]);
+                    if (d < md) {
+                        md = d;
+                        mc = c;
+                    }
+                }
+#pragma unroll
+                for (int o = 32; o > 0; o >>= 1) {
+                    const float od = __shfl_xor(md, o);
+                    const int oc = __shfl_xor(mc, o);
+                    if (od < md || (od == md && oc < mc)) {
+                        md = od;
+                        mc = oc;
+                    }
+                }
+                if (lane == at) best = md < INFINITY ? mc : 0;
+            }
+            if (valid) a.codes[i * a.stages + a.stage0 + s] = (uint16_t)best;
+            if (a.stage0 + s + 1 < a.stages) {
+                const float4 e0 = bk[2 * best], e1 = bk[2 * best + 1];
+                const float e[8] = { e0.x, e0.y, e0.z, e0.w, e1.x, e1.y, e1.z, e1.w };
+#pragma unroll
+                for (int j = 0; j < 8; j++) v[j] = __fsub_rn(v[j], e[j]);
+            }
+        }
+        if (a.dst && valid) {
+            float4 *dst = (float4 *)(a.dst + i * 8);
+            dst[0] = make_float4(v[0], v[1], v[2], v[3]);
+            dst[1] = make_float4(v[4], v[5], v[6], v[7]);
+        }
+        if (PIECES) break;
     }
 }
 
@@ -5645,13 +5907,28 @@ extern "C" int wk_vq_encode(const float *X, long n, const float *books, int stag
                             uint16_t *codes, void *stream) {
     if (n <= 0 || stages < 1 || entries < 1 || entries > 4096) return -1;
     if (((uintptr_t)X | (uintptr_t)books | (uintptr_t)cur) & 15) return -1;
-    const size_t lds = (size_t)entries * 8 * sizeof(float);
-    static std::atomic<uint64_t> attr{0};
-    if (int r_ = lds_limit((const void *)k_vq_encode_stage, 4096 * 8 * (int)sizeof(float), attr, stream)) return r_;
-    const unsigned grid = (unsigned)((n + ENC_NT - 1) / ENC_NT);
-    for (int s = 0; s < stages; s++) {
-        hipLaunchKernelGGL(k_vq_encode_stage, dim3(grid), dim3(ENC_NT), lds, (hipStream_t)stream, X, cur,
-                           books + (size_t)s * entries * 8, entries, n, s, stages, codes);
+    static std::atomic<uint64_t> attr0{0}, attr1{0};
+    if (int r_ = lds_limit((const void *)k_vq_encode<false>, (ENC_TILES + 24) * 1024, attr0, stream)) return r_;
+    if (int r_ = lds_limit((const void *)k_vq_encode<true>, (ENC_PIECE + 48) * 1024, attr1, stream)) return r_;
+    const int nt = (entries + 15) / 16;
+    const bool pieces = nt > ENC_PIECE;
+    const int per = pieces ? 1 : min(ENC_STAGES, max(1, ENC_TILES / nt));
+    const long tiles = (n + 63) / 64;
+    // 16 waves a CU: two blocks of 8 (whose waves outlive their staging by
+    // several tiles) or, in pieces, one of 16; of 4 where there are fewer
+    // tiles than that (20,001 vectors, 2 x 4,096: 152 us; the scan 1,079)
+    const int nw = tiles < 2048 ? 4 : pieces ? 16 : 8;
+    const long blocks = (tiles + nw - 1) / nw;
+    const unsigned grid = (unsigned)(pieces ? blocks : min(blocks, 512L));
+    for (int s = 0; s < stages; s += per) {
+        const int nst = min(per, stages - s);
+        EncArgs a = { s == 0 ? X : cur, s + nst < stages ? cur : nullptr, books + (size_t)s * entries * 8, n,
+                      entries, nst, s, stages, codes };
+        const size_t lds = (size_t)((pieces ? ENC_PIECE : nst * nt) + 3 * nw) * 1024;
+        if (pieces)
+            hipLaunchKernelGGL(k_vq_encode<true>, dim3(grid), dim3(nw * 64), lds, (hipStream_t)stream, a);
+        else
+            hipLaunchKernelGGL(k_vq_encode<false>, dim3(grid), dim3(nw * 64), lds, (hipStream_t)stream, a);
         CHECK_LAUNCH();
     }
     return 0;
