@@ -2149,7 +2149,7 @@ static int chunk_experts(warp_hip_ctx *c, int layer, const layer_t *B, const flo
     KRN(c, wait_copies(c));
     KRN(c, wk_plan_chunk(c->idx, c->w, T, K, E, table, c->counts, c->offsets, c->pair_tok, c->pair_exp, c->pair_w,
                          c->tok_slots, c->jobs, c->max_jobs, c->njobs, c->runs, c->missing, I, e_lo, e_hi, !first,
-                         c->st));
+                         prefill_fp16(c) ? WARP_RUN_J : WARP_RUN_JX, c->st));
     DEV(c, hipEventRecord(c->ev_before, c->st));
     float *yk[3] = { c->yg, c->yu, c->yd };
     if (c->P6) {
@@ -2163,7 +2163,7 @@ static int chunk_experts(warp_hip_ctx *c, int layer, const layer_t *B, const flo
         KRN(c, wk_apply_p6(c->jobs, c->njobs, c->max_jobs, 2, 1, P, c->lut8d, c->lscaled, P, yk + 2, H, I, c->n_cu,
                            c->st));
     } else {
-        /* by runs: each expert's records decoded once per WARP_RUN_J jobs */
+        /* by runs: each expert's records decoded once per run's jobs */
         if (prefill_fp16(c)) {
             /* reduced precision: inputs by pair slot, position-group-major
              * (x replicated per pair once the first plan has placed them) */

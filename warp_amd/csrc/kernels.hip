@@ -2600,12 +2600,12 @@ struct VqArgs {
     unsigned *queue;            // run kernels: per kind, a ticket and a waves-done counter
 };
 
-// Units of the run kernels are dealt in chunks of NW consecutive units (a
-// block's waves) to RQ_GROUPS queues, one per XCD (blocks go to the XCDs
-// round-robin, which matters only for speed: the queues are correct
+// Units of the run kernels are dealt in chunks of nw consecutive units (a
+// block's working waves) to RQ_GROUPS queues, one per XCD (blocks go to the
+// XCDs round-robin, which matters only for speed: the queues are correct
 // wherever the blocks run; the grid is a multiple of RQ_GROUPS): queue g holds
 // chunks g, g + 8, g + 16, ... and serves blocks g, g + 8, .... A wave's
-// first unit is its block's own chunk (block b, wave w: unit b NW + w);
+// first unit is its block's own chunk (block b, wave w: unit b nw + w);
 // after each unit it takes a ticket from its queue, so a wave that finishes
 // early takes the next unit of its queue, and the last, partial round
 // spreads over the CUs instead of falling on the waves of the first blocks.
@@ -2616,28 +2616,32 @@ struct VqArgs {
 // (RQ_LINE words a line) and a waves-done counter on the next line; the
 // last wave of the group out clears both, so every launch (graph replays
 // included) starts from zero without a memset.
+// nw, the waves of a block that work, is as few as give every unit a wave
+// at once, up to all of them: a launch of few units spreads over the CUs.
 constexpr int RQ_LINE = 32, RQ_GROUPS = 8;
 
 struct RunQueue {
     unsigned *q;                // the ticket counter; waves done one line on
     int n;                      // units of this queue
+    int nw;                     // working waves per block
     int nwaves;                 // waves of this queue's blocks
 };
 
 template <int NW> __device__ __forceinline__ RunQueue rq_open(unsigned *base, int kind, int units) {
-    constexpr int span = NW * RQ_GROUPS;
     const int g = blockIdx.x % RQ_GROUPS;
     RunQueue r;
-    r.n = (units / span) * NW + min(max(units % span - g * NW, 0), NW);
-    r.nwaves = (int)(gridDim.x / RQ_GROUPS) * NW;
+    r.nw = min(max((units + (int)gridDim.x - 1) / (int)gridDim.x, 1), NW);
+    const int span = r.nw * RQ_GROUPS;
+    r.n = (units / span) * r.nw + min(max(units % span - g * r.nw, 0), r.nw);
+    r.nwaves = (int)(gridDim.x / RQ_GROUPS) * r.nw;
     r.q = base + 2 * (kind * RQ_GROUPS + g) * RQ_LINE;
     return r;
 }
 
 // this block's first local index, and local index l of its queue -> unit
-template <int NW> __device__ __forceinline__ int rq_first() { return (int)(blockIdx.x / RQ_GROUPS) * NW; }
-template <int NW> __device__ __forceinline__ int rq_unit(int l) {
-    return (l / NW) * NW * RQ_GROUPS + (int)(blockIdx.x % RQ_GROUPS) * NW + l % NW;
+__device__ __forceinline__ int rq_first(const RunQueue &r) { return (int)(blockIdx.x / RQ_GROUPS) * r.nw; }
+__device__ __forceinline__ int rq_unit(const RunQueue &r, int l) {
+    return (l / r.nw) * r.nw * RQ_GROUPS + (int)(blockIdx.x % RQ_GROUPS) * r.nw + l % r.nw;
 }
 
 __device__ __forceinline__ int rq_take(const RunQueue &r, int lane) {
@@ -2857,147 +2861,196 @@ static int launch_vq_t(const VqArgs &a, int nkinds, int max_units, int npg, int 
 }
 
 // Prefill by runs: one wave per (run, 64-row block), a run being up to
-// WARP_RUN_J consecutive jobs of one expert (up to 32 of its tokens, from
+// WARP_RUN_JX consecutive jobs of one expert (up to 16 of its tokens, from
 // the grouping's run list; njobs[3] runs). The wave gathers the expert's
 // codebook vectors (the A operands) once per position group and multiplies
-// them with the B operands of every job of the run, so a busy expert's
-// records are decoded once per 32 tokens instead of once per 8; only the
-// run's own jobs are multiplied. No split over positions: the wave walks
-// all of a unit's positions, the next group's gathers issued before the
-// current group's MFMAs, then writes its rows (8 waves per block, so each
-// holds 4 x 4 accumulator tiles). Code words stream from HBM WD groups
-// ahead (8 waves per CU need that many bytes in flight); the B operands
-// come from L2, BD groups ahead.
-template <int FMT, int WD>
-__global__ __launch_bounds__(512) void k_vq_mfma_run(VqArgs a, const int *__restrict__ runs) {
+// them with the B operands of every job of the run; the loop is compiled for
+// each job count, so a run of one job loads and multiplies one. No split
+// over positions: the wave walks all of a unit's positions, then writes its
+// rows.
+//
+// What bounds it: the gathers' LDS reads (a wave's 16-byte gather takes 4
+// cycles, 16 lanes each, and as many times more as lanes of one cycle meet
+// in a column of 4 banks: 3.1 times for random entries) and, with few waves,
+// latency. So a block holds 16 waves (4 per SIMD, within 128 VGPRs: two jobs'
+// accumulators, single-buffered gathers), and the 256-entry codebooks lie in
+// LDS once per column, copy c of an entry in column c (RunBooks). The queue's
+// grid is one block per CU over all kinds of a launch.
+// 201 tokens through 256 experts of 3 x 256 codes at 2304 x 1024 (Zipf):
+// gate and up 256 -> 179 us, down 146 -> 104 (8 waves, loads and B registers
+// for four jobs whatever the run had, one copy, before); 8 copies gave 204 and
+// 110, with LDS active 7.8 cycles per gather instead of 5.3. 32 tokens through
+// 384 experts of 2 x 4096 at 7168 x 2048: 1,026 -> 911 and 580 -> 474 us, LDS
+// active 93% of the time, two thirds of that in conflicts.
+//
+// A run kernel's codebooks in LDS. 4096 entries a stage: as they are. 256
+// entries: stages 0 and 1 in 16 copies each, the third stage (what is left of
+// the 160 KiB) in 8, where two lanes still share a column half the time.
+// at[s]: the lane's base for stage s.
+template <int FMT> struct RunBooks {
     typedef FmtT<FMT> F;
-    constexpr int RJ = WARP_RUN_J;
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds_vq[];
-    const int kind = a.kind_lo + blockIdx.y;
-    const warp_job *jobs = a.jobs + (size_t)kind * a.max_jobs;
-    const int M = a.M, N = a.N, nv = N >> 3, npg = nv >> 2, nrb = (M + 63) >> 6;
-    const RunQueue rq = rq_open<8>(a.queue, kind, a.njobs[3] * nrb);
-    if (rq_first<8>() >= rq.n) {                    // uniform per block
-        rq_leave(rq, threadIdx.x, 8);
-        return;
+    static constexpr bool REP = F::E == 256;
+    static constexpr int VECS = REP ? 256 * (F::S == 3 ? 40 : 32) : F::S * F::E;   // 16-byte vectors
+    const unsigned char *at[F::S];
+    static __device__ __forceinline__ void stage(uint4 *dst, const uint16_t *books) {
+        const uint4 *src = (const uint4 *)books;
+        for (int i = threadIdx.x; i < VECS; i += blockDim.x)
+            dst[i] = src[!REP ? i : i < 8192 ? i >> 4 : 512 + ((i - 8192) >> 3)];
     }
-    {
-        const uint4 *src = (const uint4 *)(a.books + (size_t)kind * F::S * F::E * 8);
-        uint4 *dst = (uint4 *)lds_vq;
-        for (int i = threadIdx.x; i < F::S * F::E; i += blockDim.x) dst[i] = src[i];
+    __device__ __forceinline__ RunBooks(const uint4 *lds, int lane) {
+#pragma unroll
+        for (int s = 0; s < F::S; s++)
+            at[s] = (const unsigned char *)lds + (!REP ? s * 65536 : s * 65536 + 16 * (lane & (s < 2 ? 15 : 7)));
     }
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int g = lane >> 4, jc = lane & 15, ts = jc >> 1, hl = jc & 1;
-    for (int l = rq_first<8>() + wave; l < rq.n;) {
-        const int u = rq_unit<8>(l);
-        const int rv = __builtin_amdgcn_readfirstlane(runs[u / nrb]);   // uniform: u is
-        const int j0 = rv >> 3, nt = rv & 7, rb = u % nrb;
-        const uint8_t *cp = jobs[j0].idx + ((size_t)rb * nv) * 64 * F::SB + (size_t)lane * 4 * F::SB;
-        // B operands of every job of the run; a slot past a job's tokens
-        // points at one of its tokens (the grouping fills every slot), so
-        // every load is unconditional: its column of the product is not
-        // written out. Loads without branches keep the wait counts exact.
-        const _Float16 *xrow[RJ];
+    // the vectors of 4 consecutive rows at one position
+    __device__ __forceinline__ void gather(const Word<F::SB> &wd, half8 (&a)[4][F::S]) const {
 #pragma unroll
-        for (int q = 0; q < RJ; q++)
-            xrow[q] = a.xs + (size_t)jobs[j0 + min(q, nt - 1)].xi[ts] * nv * 16 + hl * 8 + (size_t)g * 16;
-        f4 acc[RJ][4];
+        for (int t = 0; t < 4; t++) {
+            const unsigned sl = wd.slot(t);
 #pragma unroll
-        for (int q = 0; q < RJ; q++)
-#pragma unroll
-            for (int t = 0; t < 4; t++) acc[q][t] = f4{0.f, 0.f, 0.f, 0.f};
-        constexpr int BD = 2;
-        Word<F::SB> buf[WD];
-        half8 bb[BD][RJ];
-#pragma unroll
-        for (int k = 0; k < WD; k++) buf[k].load_keep(cp + (size_t)min(k, npg - 1) * 256 * F::SB);
-#pragma unroll
-        for (int k = 0; k < BD; k++)
-#pragma unroll
-            for (int q = 0; q < RJ; q++) bb[k][q] = *(const half8 *)(xrow[q] + (size_t)min(k, npg - 1) * 64);
-        half8 av[2][4][F::S];
-        gather_group<FMT, F::SB>(lds_vq, buf[0], av[0]);
-        // one position group: the next group's gathers, the loads WD (code
-        // words) and BD (B) groups ahead, clamped to the last group, then
-        // this group's MFMAs
-        auto step = [&](int k, int pg) {
-            const int cur = k & 1;                            // = pg & 1: WD is even
-            half8 b[RJ];
-#pragma unroll
-            for (int q = 0; q < RJ; q++) b[q] = bb[k % BD][q];
-            gather_group<FMT, F::SB>(lds_vq, buf[(k + 1) % WD], av[cur ^ 1]);
-            buf[k].load_keep(cp + (size_t)min(pg + WD, npg - 1) * 256 * F::SB);
-#pragma unroll
-            for (int q = 0; q < RJ; q++) bb[k % BD][q] = *(const half8 *)(xrow[q] + (size_t)min(pg + BD, npg - 1) * 64);
-            // stage-major: the 4 row tiles' chains interleave, no MFMA waits on the previous one
-#pragma unroll
-            for (int q = 0; q < RJ; q++)
-                if (q < nt)                                   // uniform
-#pragma unroll
-                    for (int s = 0; s < F::S; s++)
-#pragma unroll
-                        for (int t = 0; t < 4; t++)
-                            acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[cur][t][s], b[q], acc[q][t], 0, 0, 0);
-        };
-        const int npg_full = npg - npg % WD;
-        for (int pgb = 0; pgb < npg_full; pgb += WD) {
-#pragma unroll
-            for (int k = 0; k < WD; k++) step(k, pgb + k);
-        }
-#pragma unroll
-        for (int k = 0; k < WD; k++)
-            if (npg_full + k < npg) step(k, npg_full + k);    // uniform
-        l = rq_take(rq, lane);                                // returns while the outputs are stored
-        // lane (g, jc) holds C[4g + r][jc] of row tile t: block row 16g + 4r + t,
-        // token slot jc / 2 of the job, half jc % 2 -- the 16 consecutive rows
-        // 16g .. 16g + 15, stored as four 16-byte runs
-#pragma unroll
-        for (int q = 0; q < RJ; q++) {
-            if (q >= nt) break;                               // uniform
-            const warp_job &jq = jobs[j0 + q];
-            const bool tv = hl == 0 && ts < jq.n;
-            const float xsc = tv ? a.xscale[jq.xi[ts]] : 0.0f;
-            const int yrow = tv ? jq.yi[ts] : 0;
-            float *yo = a.y[kind] + (size_t)yrow * M;
-            if ((M & 63) == 0) {                              // uniform: whole 64-row blocks
-                // the same 4 x 4 transpose as the reduced-precision kernel's:
-                // store k writes rows 16k .. 16k + 15 as one 64-byte sector
-                float w[4][4];
-                auto pick = [](const float *u, int i) { return i == 0 ? u[0] : i == 1 ? u[1] : i == 2 ? u[2] : u[3]; };
-#pragma unroll
-                for (int t = 0; t < 4; t++) {
-                    float v[4];                               // rows 16 g + 4 r + t
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        v[r] = ((acc[q][t][r] + __shfl_xor(acc[q][t][r], 1)) * xsc) *
-                               f16_keep(jq.scale[rb * 64 + 16 * g + 4 * r + t]);
-#pragma unroll
-                    for (int d = 0; d < 4; d++) {
-                        const float sv = pick(v, g ^ d);
-                        w[d][t] = d == 0 ? sv : __shfl_xor(sv, 16 * d);
-                    }
-                }
-#pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const int d = g ^ k;
-                    const float4 o = make_float4(d == 0 ? w[0][0] : d == 1 ? w[1][0] : d == 2 ? w[2][0] : w[3][0],
-                                                 d == 0 ? w[0][1] : d == 1 ? w[1][1] : d == 2 ? w[2][1] : w[3][1],
-                                                 d == 0 ? w[0][2] : d == 1 ? w[1][2] : d == 2 ? w[2][2] : w[3][2],
-                                                 d == 0 ? w[0][3] : d == 1 ? w[1][3] : d == 2 ? w[2][3] : w[3][3]);
-                    if (tv) *(float4 *)(yo + rb * 64 + 16 * k + 4 * g) = o;
-                }
-            } else {
-#pragma unroll
-                for (int r = 0; r < 4; r++)
-#pragma unroll
-                    for (int t = 0; t < 4; t++) {
-                        const float v = acc[q][t][r] + __shfl_xor(acc[q][t][r], 1);
-                        const int row = rb * 64 + 16 * g + 4 * r + t;
-                        if (tv && row < M) yo[row] = (v * xsc) * f16_keep(jq.scale[row]);
-                    }
+            for (int s = 0; s < F::S; s++) {
+                const unsigned c = REP ? (sl >> (8 * s)) & 0xFFu : s ? sl >> 12 : sl & 0xFFFu;
+                a[t][s] = *(const half8 *)(at[s] + c * (!REP ? 16u : s < 2 ? 256u : 128u));
             }
         }
+    }
+};
+
+// one unit: the rows of block rb of the NT jobs from j0
+template <int FMT, int WD, int NT>
+__device__ __forceinline__ void run_unit(const VqArgs &a, const warp_job *jobs, float *y, int j0, int rb, int lane,
+                                         const RunBooks<FMT> &cb) {
+    typedef FmtT<FMT> F;
+    const int M = a.M, nv = a.N >> 3, npg = nv >> 2;
+    const int g = lane >> 4, jc = lane & 15, ts = jc >> 1, hl = jc & 1;
+    const uint8_t *cp = jobs[j0].idx + ((size_t)rb * nv) * 64 * F::SB + (size_t)lane * 4 * F::SB;
+    // B operands of every job of the run; a slot past a job's tokens
+    // points at one of its tokens (the grouping fills every slot), so
+    // every load is unconditional: its column of the product is not
+    // written out. Loads without branches keep the wait counts exact.
+    const _Float16 *xrow[NT];
+#pragma unroll
+    for (int q = 0; q < NT; q++) xrow[q] = a.xs + (size_t)jobs[j0 + q].xi[ts] * nv * 16 + hl * 8 + (size_t)g * 16;
+    f4 acc[NT][4];
+#pragma unroll
+    for (int q = 0; q < NT; q++)
+#pragma unroll
+        for (int t = 0; t < 4; t++) acc[q][t] = f4{0.f, 0.f, 0.f, 0.f};
+    Word<F::SB> buf[WD];
+    half8 bb[WD][NT];
+#pragma unroll
+    for (int k = 0; k < WD; k++) {
+        const int pk = min(k, npg - 1);
+        buf[k].load_keep(cp + (size_t)pk * 256 * F::SB);
+#pragma unroll
+        for (int q = 0; q < NT; q++) bb[k][q] = *(const half8 *)(xrow[q] + (size_t)pk * 64);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // one position group: its gathers, the code word WD groups ahead (clamped
+    // to the last group), its MFMAs, then B WD groups ahead into the
+    // registers that the MFMAs have read
+    auto step = [&](int k, int pg) {
+        half8 av[4][F::S];
+        cb.gather(buf[k], av);
+        const int pn = min(pg + WD, npg - 1);
+        buf[k].load_keep(cp + (size_t)pn * 256 * F::SB);
+        // stage-major: the 4 row tiles' chains interleave, no MFMA waits on the previous one
+#pragma unroll
+        for (int s = 0; s < F::S; s++)
+#pragma unroll
+            for (int q = 0; q < NT; q++)
+#pragma unroll
+                for (int t = 0; t < 4; t++)
+                    acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[t][s], bb[k][q], acc[q][t], 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < NT; q++) bb[k][q] = *(const half8 *)(xrow[q] + (size_t)pn * 64);
+        // (the loads stay in their step, here and before the loop: left alone,
+        // the scheduler collects them at the end of the unrolled body, just
+        // before their first wait)
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const int npg_full = npg - npg % WD;
+    for (int pgb = 0; pgb < npg_full; pgb += WD) {
+#pragma unroll
+        for (int k = 0; k < WD; k++) step(k, pgb + k);
+    }
+#pragma unroll
+    for (int k = 0; k < WD; k++)
+        if (npg_full + k < npg) step(k, npg_full + k);    // uniform
+    // lane (g, jc) holds C[4g + r][jc] of row tile t: block row 16g + 4r + t,
+    // token slot jc / 2 of the job, half jc % 2 -- the 16 consecutive rows
+    // 16g .. 16g + 15, stored as four 16-byte runs
+#pragma unroll
+    for (int q = 0; q < NT; q++) {
+        const warp_job &jq = jobs[j0 + q];
+        const bool tv = hl == 0 && ts < jq.n;
+        const float xsc = tv ? a.xscale[jq.xi[ts]] : 0.0f;
+        const int yrow = tv ? jq.yi[ts] : 0;
+        float *yo = y + (size_t)yrow * M;
+        if ((M & 63) == 0) {                              // uniform: whole 64-row blocks
+            // the same 4 x 4 transpose as the reduced-precision kernel's:
+            // store k writes rows 16k .. 16k + 15 as one 64-byte sector
+            float w[4][4];
+            auto pick = [](const float *u, int i) { return i == 0 ? u[0] : i == 1 ? u[1] : i == 2 ? u[2] : u[3]; };
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                float v[4];                               // rows 16 g + 4 r + t
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    v[r] = ((acc[q][t][r] + __shfl_xor(acc[q][t][r], 1)) * xsc) *
+                           f16_keep(jq.scale[rb * 64 + 16 * g + 4 * r + t]);
+#pragma unroll
+                for (int d = 0; d < 4; d++) {
+                    const float sv = pick(v, g ^ d);
+                    w[d][t] = d == 0 ? sv : __shfl_xor(sv, 16 * d);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int d = g ^ k;
+                const float4 o = make_float4(d == 0 ? w[0][0] : d == 1 ? w[1][0] : d == 2 ? w[2][0] : w[3][0],
+                                             d == 0 ? w[0][1] : d == 1 ? w[1][1] : d == 2 ? w[2][1] : w[3][1],
+                                             d == 0 ? w[0][2] : d == 1 ? w[1][2] : d == 2 ? w[2][2] : w[3][2],
+                                             d == 0 ? w[0][3] : d == 1 ? w[1][3] : d == 2 ? w[2][3] : w[3][3]);
+                if (tv) *(float4 *)(yo + rb * 64 + 16 * k + 4 * g) = o;
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int t = 0; t < 4; t++) {
+                    const float v = acc[q][t][r] + __shfl_xor(acc[q][t][r], 1);
+                    const int row = rb * 64 + 16 * g + 4 * r + t;
+                    if (tv && row < M) yo[row] = (v * xsc) * f16_keep(jq.scale[row]);
+                }
+        }
+    }
+}
+
+template <int FMT, int WD1, int WD2>
+__global__ __launch_bounds__(1024) void k_vq_mfma_run(VqArgs a, const int *__restrict__ runs) {
+    typedef FmtT<FMT> F;
+    __shared__ uint4 cb_lds[RunBooks<FMT>::VECS];
+    const int kind = a.kind_lo + blockIdx.y;
+    const warp_job *jobs = a.jobs + (size_t)kind * a.max_jobs;
+    const int nrb = (a.M + 63) >> 6;
+    const RunQueue rq = rq_open<16>(a.queue, kind, a.njobs[3] * nrb);
+    if (rq_first(rq) >= rq.n) {                     // uniform per block
+        rq_leave(rq, threadIdx.x, rq.nw);
+        return;
+    }
+    RunBooks<FMT>::stage(cb_lds, a.books + (size_t)kind * F::S * F::E * 8);
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (wave >= rq.nw) return;
+    const RunBooks<FMT> cb(cb_lds, lane);
+    for (int l = rq_first(rq) + wave; l < rq.n;) {
+        const int u = rq_unit(rq, l);
+        const int rv = __builtin_amdgcn_readfirstlane(runs[u / nrb]);   // uniform: u is
+        static_assert(WARP_RUN_JX == 2, "a loop per job count");
+        if ((rv & 7) == 1) run_unit<FMT, WD1, 1>(a, jobs, a.y[kind], rv >> 3, u % nrb, lane, cb);
+        else run_unit<FMT, WD2, 2>(a, jobs, a.y[kind], rv >> 3, u % nrb, lane, cb);
+        l = rq_take(rq, lane);
     }
     rq_leave(rq, lane, 1);
 }
@@ -3005,15 +3058,12 @@ __global__ __launch_bounds__(512) void k_vq_mfma_run(VqArgs a, const int *__rest
 template <int FMT>
 static int launch_vq_run(const VqArgs &a, const int *runs, int nkinds, int max_units, void *stream) {
     typedef FmtT<FMT> F;
-    constexpr int WD = F::S == 3 ? 2 : 8;                   // three stages leave room for fewer words
-    const size_t lds = (size_t)F::S * F::E * 16;
-    static std::atomic<uint64_t> attr{0};
-    if (int r_ = lds_limit((const void *)k_vq_mfma_run<FMT, WD>, (int)lds, attr, stream)) return r_;
-    int grid = (max_units + 7) / 8;
-    const int cap = FMT == WARP_FMT_VQ12 ? 256 : 1024;
-    if (grid > cap) grid = cap;
+    constexpr int WD1 = F::S == 3 ? 4 : 6, WD2 = F::S == 3 ? 2 : 3;
+    // one block per CU: the kinds of a launch share the CUs
+    int grid = 256 / nkinds;
+    if (grid > max_units) grid = max_units;
     grid = (grid + RQ_GROUPS - 1) / RQ_GROUPS * RQ_GROUPS;   // the unit queues' groups
-    hipLaunchKernelGGL((k_vq_mfma_run<FMT, WD>), dim3(grid, nkinds), dim3(512), lds, (hipStream_t)stream, a, runs);
+    hipLaunchKernelGGL((k_vq_mfma_run<FMT, WD1, WD2>), dim3(grid, nkinds), dim3(1024), 0, (hipStream_t)stream, a, runs);
     CHECK_LAUNCH();
     return 0;
 }
@@ -3045,30 +3095,27 @@ template <int FMT, int WD>
 __global__ __launch_bounds__(1024) void k_vq_run_f16(VqArgs a, const int *__restrict__ runs) {
     typedef FmtT<FMT> F;
     constexpr int NWB = 16, RB = WARP_RUN_J / 2;            // waves per block; B operands (2 jobs each) per step
-    // the codebook at a fixed LDS address, so the gathers' addresses need no base
-    __shared__ uint4 cb_lds[F::S * F::E];
-    const unsigned char *lds_vq = (const unsigned char *)cb_lds;
+    __shared__ uint4 cb_lds[RunBooks<FMT>::VECS];
     const int kind = a.kind_lo + blockIdx.y;
     const warp_job *jobs = a.jobs + (size_t)kind * a.max_jobs;
     const int M = a.M, N = a.N, nv = N >> 3, npg = nv >> 2, nrb = (M + 63) >> 6;
     const RunQueue rq = rq_open<NWB>(a.queue, kind, a.njobs[3] * nrb);
-    if (rq_first<NWB>() >= rq.n) {                  // uniform per block
-        rq_leave(rq, threadIdx.x, NWB);
+    if (rq_first(rq) >= rq.n) {                  // uniform per block
+        rq_leave(rq, threadIdx.x, rq.nw);
         return;
     }
-    {
-        const uint4 *src = (const uint4 *)(a.books + (size_t)kind * F::S * F::E * 8);
-        for (int i = threadIdx.x; i < F::S * F::E; i += blockDim.x) cb_lds[i] = src[i];
-    }
+    RunBooks<FMT>::stage(cb_lds, a.books + (size_t)kind * F::S * F::E * 8);
     __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (wave >= rq.nw) return;
+    const RunBooks<FMT> cb(cb_lds, lane);
     const int g = lane >> 4, jc = lane & 15;
     // B and the code words through buffer loads: a per-lane offset fixed for
     // the unit and a per-group offset in a scalar register
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void *)a.xs, 0, -1, BUF_RSRC_W3);
     const int pgb_x = a.xrows * 64;                          // bytes per position group of xs
-    for (int l = rq_first<NWB>() + wave; l < rq.n;) {
-        const int u = rq_unit<NWB>(l);
+    for (int l = rq_first(rq) + wave; l < rq.n;) {
+        const int u = rq_unit(rq, l);
         const int rv = __builtin_amdgcn_readfirstlane(runs[u / nrb]);   // uniform: u is
         const int j0 = rv >> 3, nt = rv & 7, rb = u % nrb;
         // the unit's code words (uniform: the descriptor lives in scalar registers)
@@ -3102,13 +3149,14 @@ __global__ __launch_bounds__(1024) void k_vq_run_f16(VqArgs a, const int *__rest
 #pragma unroll
             for (int q = 0; q < RB; q++)
                 bb[k][q] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(xr, xo[q], pk * pgb_x, 0));
+            __builtin_amdgcn_sched_barrier(0);
         }
         // one position group: its gathers, the code word WD groups ahead,
         // the stage sums and MFMAs, then B WD groups ahead into the slot the
         // MFMAs have read
         auto step = [&](int k, int pg) {
             half8 av[4][F::S];
-            gather_group<FMT, F::SB>(lds_vq, buf[k], av);
+            cb.gather(buf[k], av);
             const int pn = min(pg + WD, npg - 1);
             word_load<F::SB>(buf[k], cr, co, pn * 256 * F::SB);
 #pragma unroll
@@ -3124,6 +3172,7 @@ __global__ __launch_bounds__(1024) void k_vq_run_f16(VqArgs a, const int *__rest
 #pragma unroll
             for (int q = 0; q < RB; q++)
                 bb[k][q] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(xr, xo[q], pn * pgb_x, 0));
+            __builtin_amdgcn_sched_barrier(0);                // (the loads stay in their step)
         };
         const int npg_full = npg - npg % WD;
         for (int pgb = 0; pgb < npg_full; pgb += WD) {
@@ -3194,9 +3243,8 @@ template <int FMT>
 static int launch_vq_run_f16(const VqArgs &a, const int *runs, int nkinds, int max_units, void *stream) {
     typedef FmtT<FMT> F;
     constexpr int WD = F::S == 3 ? 2 : 3;                   // code words and B operands in flight
-    int grid = (max_units + 15) / 16;
-    const int cap = FMT == WARP_FMT_VQ12 ? 256 : 512;
-    if (grid > cap) grid = cap;
+    int grid = 256 / nkinds;                                // one block per CU: the kinds share the CUs
+    if (grid > max_units) grid = max_units;
     grid = (grid + RQ_GROUPS - 1) / RQ_GROUPS * RQ_GROUPS;   // the unit queues' groups
     hipLaunchKernelGGL((k_vq_run_f16<FMT, WD>), dim3(grid, nkinds), dim3(1024), 0, (hipStream_t)stream, a, runs);
     CHECK_LAUNCH();
@@ -5292,7 +5340,7 @@ __global__ __launch_bounds__(1024) void k_plan_chunk(const int *__restrict__ idx
                                                      warp_job *__restrict__ jobs, int max_jobs,
                                                      int *__restrict__ njobs, int *__restrict__ runs,
                                                      int *__restrict__ missing, int inter, int bitmaps,
-                                                     int e_lo, int e_hi, int or_missing) {
+                                                     int e_lo, int e_hi, int or_missing, int run_j) {
     extern __shared__ __attribute__((aligned(16))) int lds_plan[];
     // token bitmap rows of NWP words: an odd stride, so the rows that a
     // wave's pairs read in one step fall on different LDS banks
@@ -5355,7 +5403,7 @@ __global__ __launch_bounds__(1024) void k_plan_chunk(const int *__restrict__ idx
     }
     __syncthreads();
     // per expert, in parallel: pair offset, first job, and the places of
-    // its runs -- heaviest first: every full run of WARP_RUN_J jobs, then the
+    // its runs -- heaviest first: every full run of run_j jobs, then the
     // partial runs by their job count down to 1 (the launch hands units to
     // waves round-robin, so the long ones start first)
     __shared__ unsigned long long sc_tmp[16];
@@ -5368,13 +5416,13 @@ __global__ __launch_bounds__(1024) void k_plan_chunk(const int *__restrict__ idx
         const int e = e0 + threadIdx.x;
         // every pair gets its place; jobs and runs only the window's experts
         const int c = e < E ? cnt[e] : 0, cw = e >= e_lo && e <= e_hi ? c : 0;
-        const int nt = (cw + WARP_TPJ - 1) / WARP_TPJ, r = nt % WARP_RUN_J;
+        const int nt = (cw + WARP_TPJ - 1) / WARP_TPJ, r = nt % run_j;
         // pairs, jobs and full runs in one scan; the partial runs of 1, 2
         // and 3 jobs in another
         unsigned long long t0, t1;
         const unsigned long long s0 =
             block_scan_excl64((unsigned long long)c | ((unsigned long long)nt << 21) |
-                                  ((unsigned long long)(nt / WARP_RUN_J) << 42), sc_tmp, t0);
+                                  ((unsigned long long)(nt / run_j) << 42), sc_tmp, t0);
         const unsigned long long s1 =
             block_scan_excl64((unsigned long long)(r == 1) | ((unsigned long long)(r == 2) << 21) |
                                   ((unsigned long long)(r == 3) << 42), sc_tmp, t1);
@@ -5407,7 +5455,7 @@ __global__ __launch_bounds__(1024) void k_plan_chunk(const int *__restrict__ idx
     for (int q = WARP_RUN_J - 1; q > 1; q--) base[q - 1] = base[q] + carry[2 + q];
     for (int e = threadIdx.x; e < E; e += blockDim.x) {
         const int cw = e >= e_lo && e <= e_hi ? cnt[e] : 0;
-        const int r = ((cw + WARP_TPJ - 1) / WARP_TPJ) % WARP_RUN_J;
+        const int r = ((cw + WARP_TPJ - 1) / WARP_TPJ) % run_j;
 #pragma unroll
         for (int q = 1; q < WARP_RUN_J; q++)
             if (r == q) runr[e] += base[q];
@@ -5467,10 +5515,10 @@ __global__ __launch_bounds__(1024) void k_plan_chunk(const int *__restrict__ idx
     // the runs, one thread per expert (a few entries each)
     for (int e = threadIdx.x; e < E; e += blockDim.x) {
         const int ntile = e >= e_lo && e <= e_hi ? (cnt[e] + WARP_TPJ - 1) / WARP_TPJ : 0;
-        for (int i = 0; i + WARP_RUN_J <= ntile; i += WARP_RUN_J)
-            runs[run0[e] + i / WARP_RUN_J] = ((tile0[e] + i) << 3) | WARP_RUN_J;
-        if (ntile % WARP_RUN_J)
-            runs[runr[e]] = ((tile0[e] + ntile / WARP_RUN_J * WARP_RUN_J) << 3) | (ntile % WARP_RUN_J);
+        const int part = ntile % run_j, full = ntile - part;
+        int *ro = runs + run0[e];
+        for (int i = 0; i < full; i += run_j) *ro++ = ((tile0[e] + i) << 3) | run_j;
+        if (part) runs[runr[e]] = ((tile0[e] + full) << 3) | part;
     }
     // the jobs, one thread per job: its expert is the last one whose first
     // job is not after it (experts without jobs share the next one's first)
@@ -5510,8 +5558,10 @@ __global__ __launch_bounds__(1024) void k_plan_chunk(const int *__restrict__ idx
 extern "C" int wk_plan_chunk(const int *idx, const float *w, int T, int K, int E, const warp_slot *table,
                              int *counts, int *offsets, int *pair_tok, int *pair_exp, float *pair_w, int *tok_slots,
                              warp_job *jobs, int max_jobs, int *njobs, int *runs, int *missing, int inter,
-                             int e_lo, int e_hi, int or_missing, void *stream) {
-    if (T <= 0 || K <= 0 || E <= 0 || max_jobs <= 0 || !runs || e_lo < 0 || e_hi >= E || e_lo > e_hi) return -1;
+                             int e_lo, int e_hi, int or_missing, int run_j, void *stream) {
+    if (T <= 0 || K <= 0 || E <= 0 || max_jobs <= 0 || !runs || e_lo < 0 || e_hi >= E || e_lo > e_hi || run_j < 1 ||
+        run_j > WARP_RUN_J)
+        return -1;
     // the picks, the per-expert tables, each pair's token and a flag per pair
     // in LDS; the token bitmaps too when they fit
     const size_t base = (size_t)E * sizeof(warp_slot) + ((size_t)2 * T * K + 5 * (size_t)E) * sizeof(int) +
@@ -5525,7 +5575,7 @@ extern "C" int wk_plan_chunk(const int *idx, const float *w, int T, int K, int E
     if (int r_ = lds_limit((const void *)k_plan_chunk, (int)LDS_MAX, attr, stream)) return r_;
     hipLaunchKernelGGL(k_plan_chunk, dim3(1), dim3(1024), base + (bitmaps ? bms : 0), (hipStream_t)stream, idx, w, T,
                        K, E, table, counts, offsets, pair_tok, pair_exp, pair_w, tok_slots, jobs, max_jobs, njobs,
-                       runs, missing, inter, bitmaps, e_lo, e_hi, or_missing);
+                       runs, missing, inter, bitmaps, e_lo, e_hi, or_missing, run_j);
     CHECK_LAUNCH();
     return 0;
 }

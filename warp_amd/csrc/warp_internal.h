@@ -35,7 +35,8 @@ extern "C" {
 #define WARP_TILE 64          /* index_block of the container format     */
 #define WARP_LUT_BLK 32       /* positions per int8 LUT scale (VQ4P)     */
 #define WARP_TPJ 8            /* token slots per matvec job              */
-#define WARP_RUN_J 4          /* jobs of one expert per prefill run      */
+#define WARP_RUN_J 4          /* most jobs of one expert per prefill run */
+#define WARP_RUN_JX 2         /* the same for exact products             */
 #define WARP_MAX_K 64         /* top-k bound (the reference's cfg_sane)  */
 
 /* One matvec job: one matrix (kind) of one expert record against up to
@@ -174,8 +175,8 @@ int wk_vq_matvec(int fmt, const warp_job *jobs, const int *njobs, int max_jobs,
                  const float *xscale, float *const *y, int M, int N, int tokens_per_job,
                  void *stream);
 /* The same for prefill by runs: runs[0..njobs[3]) = (first job << 3) | jobs,
- * up to WARP_RUN_J consecutive jobs of one expert (wk_plan_chunk writes
- * them); each run's records are decoded once for all its jobs.
+ * up to WARP_RUN_J (exact products: WARP_RUN_JX) consecutive jobs of one
+ * expert (wk_plan_chunk writes them); each run's records are decoded once for all its jobs.
  * fp16_rows = 0: exact products, xs/xscale as for wk_vq_matvec (rows by
  * xi). fp16_rows > 0: the reduced-precision products (stage vectors added
  * in fp16, x's fp16 high half), xs [N/32][fp16_rows][32] and xscale
@@ -341,7 +342,7 @@ int wk_act(const float *g, const float *u, int P, int I, int act_situ, float bet
  * slots in ascending expert id; gate/up jobs (tiles of WARP_TPJ tokens of
  * one expert; xi = token, yi = pair slot) and down jobs (xi = yi = pair
  * slot) written to jobs[kind*max_jobs ..], counts to njobs[0..3); the runs
- * of up to WARP_RUN_J jobs of one expert to runs, their count to njobs[3].
+ * of up to run_j (<= WARP_RUN_J) jobs of one expert to runs, their count to njobs[3].
  * *missing is written every call: 1 when a pair's expert has no resident
  * record, 2 when the jobs exceed max_jobs, else 0 (with or_missing, only a
  * nonzero value is written). Jobs and runs are made for the experts
@@ -352,7 +353,7 @@ int wk_plan_chunk(const int *idx, const float *w, int T, int K, int E,
                   const warp_slot *table, int *counts, int *offsets, int *pair_tok,
                   int *pair_exp, float *pair_w, int *tok_slots, warp_job *jobs,
                   int max_jobs, int *njobs, int *runs, int *missing, int inter,
-                  int e_lo, int e_hi, int or_missing, void *stream);
+                  int e_lo, int e_hi, int or_missing, int run_j, void *stream);
 /* out [T][H] = per token, sum over its pairs in ascending expert id (tok_slots)
  * of w * y[pair], then + add0 [T][H] when given. */
 int wk_combine_chunk(const float *y, const int *tok_slots, const float *pair_w, int T, int K, int H,
