@@ -1639,14 +1639,12 @@ static int cert_ok(const warp_hip_ctx *c, const layer_t *L)
            g->hidden % 4 == 0 && g->hidden <= 16384 && g->n_experts <= 4096;
 }
 
-/* The layer's shared expert as the fused decode kernels take it: an fp32
- * router with the fast (tree) sum or the certifying one, the hidden state
- * in shh. */
-static int shared_args(const warp_hip_ctx *c, const layer_t *L, warp_shared_args *sa)
+/* The layer's shared expert as the kernels that make its hidden state (in
+ * shh) in one launch take it. */
+static void shared_mats(const warp_hip_ctx *c, const layer_t *L, warp_shared_args *sa)
 {
     const warp_hip_cfg *g = &c->cfg;
     memset(sa, 0, sizeof *sa);
-    if (!L->sq[0] || !L->router || (g->router_strict && !cert_ok(c, L)) || !c->shh) return 0;
     for (int k = 0; k < 3; k++) {
         sa->q[k] = L->sq[k];
         sa->s[k] = L->ss[k];
@@ -1659,7 +1657,14 @@ static int shared_args(const warp_hip_ctx *c, const layer_t *L, warp_shared_args
     sa->beta = g->situ_beta;
     sa->lbeta = g->situ_linear_beta;
     sa->h = c->shh;
-    return 1;
+}
+
+/* The same for the fused decode kernels: an fp32 router with the fast (tree)
+ * sum or the certifying one. */
+static int shared_args(const warp_hip_ctx *c, const layer_t *L, warp_shared_args *sa)
+{
+    shared_mats(c, L, sa);
+    return L->sq[0] && L->router && (!c->cfg.router_strict || cert_ok(c, L)) && c->shh;
 }
 
 /* The shared expert of T tokens into sho, on stream s; it touches only the
@@ -1688,9 +1693,15 @@ static int shared_ffn(warp_hip_ctx *c, const layer_t *L, const float *x, int T, 
                            &dy, s));
         return 0;
     }
-    KRN(c, wk_mvq(L->sq[0], L->ss[0], L->s_rowbytes[0], L->s_group, L->s_bits, x, Is, H, T, c->shg, s));
-    KRN(c, wk_mvq(L->sq[1], L->ss[1], L->s_rowbytes[1], L->s_group, L->s_bits, x, Is, H, T, c->shu, s));
-    KRN(c, wk_act(c->shg, c->shu, T, Is, g->act_situ, g->situ_beta, g->situ_linear_beta, c->shh, s));
+    warp_shared_args sa;
+    shared_mats(c, L, &sa);
+    if (wk_shared_h_ok(x, H, &sa)) {
+        KRN(c, wk_shared_h(x, T, H, &sa, c->n_cu, s));
+    } else {
+        KRN(c, wk_mvq(L->sq[0], L->ss[0], L->s_rowbytes[0], L->s_group, L->s_bits, x, Is, H, T, c->shg, s));
+        KRN(c, wk_mvq(L->sq[1], L->ss[1], L->s_rowbytes[1], L->s_group, L->s_bits, x, Is, H, T, c->shu, s));
+        KRN(c, wk_act(c->shg, c->shu, T, Is, g->act_situ, g->situ_beta, g->situ_linear_beta, c->shh, s));
+    }
     KRN(c, wk_mvq(L->sq[2], L->ss[2], L->s_rowbytes[2], L->s_group, L->s_bits, c->shh, H, Is, T, c->sho, s));
     return 0;
 }

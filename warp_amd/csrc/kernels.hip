@@ -1281,6 +1281,70 @@ extern "C" int wk_router_shared(const float *W, const float *x, int E, int H, fl
     return 0;
 }
 
+// A few tokens' h = act(gate . x, up . x) of the shared expert in one launch
+// (a token per grid row), where the router launch does not make it: each wave
+// takes PW rows of gate and of up in turn, loaded one ahead as in k_mvq_fast,
+// with the same sums. Two launches of that kernel and one of k_act cost 35 us
+// at 6144 x 7168 (88 MB of Q8G) and 15 us at 1024 x 2304, most of it their
+// first loads; this one 22 and 4.7 us. PW = 2 halves the staging of x per row
+// where that still gives every CU blocks.
+template <int BITS, int MC, int PW>
+__global__ __launch_bounds__(256) void k_shared_h(const float *__restrict__ x, int H, warp_shared_args sa) {
+    extern __shared__ __attribute__((aligned(16))) float xl[];
+    using Q = QRow<BITS, MC>;
+    const int wave = threadIdx.x >> 6, nc = H / Q::WPC, ng = H / sa.group;
+    const int r0 = ((int)blockIdx.x * 4 + wave) * PW;
+    auto load = [&](Q &q, int i) {               // row i of the wave: gate, up, gate, up
+        const int r = min(r0 + (i >> 1), sa.inter - 1);
+        q.load(sa.q[i & 1] + (size_t)r * sa.rowbytes[i & 1], sa.s[i & 1] + (size_t)r * ng, sa.group, nc);
+    };
+    Q cur, nxt;
+    load(cur, 0);
+    const float *xt = x + (size_t)blockIdx.y * H;
+    for (int i = threadIdx.x; i < H / 4; i += 256) ((float4 *)xl)[i] = ((const float4 *)xt)[i];
+    __syncthreads();
+    float gv = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 2 * PW; i++) {
+        if (i + 1 < 2 * PW) load(nxt, i + 1);
+        const float v = cur.dot(xl, nc);
+        const int r = r0 + (i >> 1);
+        if (!(i & 1)) gv = v;
+        else if ((threadIdx.x & 63) == 0 && r < sa.inter)
+            sa.h[(size_t)blockIdx.y * sa.inter + r] = act_pair(gv, v, sa.situ, sa.beta, sa.lbeta);
+        if (i + 1 < 2 * PW) cur = nxt;
+    }
+}
+
+extern "C" int wk_shared_h_ok(const float *x, int H, const warp_shared_args *sa) {
+    return wk_shared_fast_ok(H, sa) && ((uintptr_t)x & 15) == 0 && (size_t)H * sizeof(float) <= 64 * 1024;
+}
+
+extern "C" int wk_shared_h(const float *x, int T, int H, const warp_shared_args *sa, int n_cu, void *stream) {
+    if (T <= 0 || !sa->h || !wk_shared_h_ok(x, H, sa)) return -1;
+    const int pw = sa->inter / 8 >= 2 * n_cu ? 2 : 1;
+    const dim3 grid((sa->inter + 4 * pw - 1) / (4 * pw), T);
+    const size_t lds = (size_t)H * sizeof(float);
+    const int mc = (H / (sa->bits == 8 ? 16 : 32) + 63) / 64;     // <= SH_MAXC (wk_shared_fast_ok)
+#define SHH(b, n)                                                                                                    \
+    do {                                                                                                             \
+        if (pw == 2) hipLaunchKernelGGL((k_shared_h<b, n, 2>), grid, dim3(256), lds, (hipStream_t)stream, x, H, *sa); \
+        else hipLaunchKernelGGL((k_shared_h<b, n, 1>), grid, dim3(256), lds, (hipStream_t)stream, x, H, *sa);        \
+    } while (0)
+    if (sa->bits == 8) {
+        if (mc <= 2) SHH(8, 2);
+        else if (mc <= 4) SHH(8, 4);
+        else SHH(8, SH_MAXC);
+    } else {
+        if (mc <= 2) SHH(4, 2);
+        else if (mc <= 4) SHH(4, 4);
+        else SHH(4, SH_MAXC);
+    }
+#undef SHH
+    CHECK_LAUNCH();
+    return 0;
+}
+
 // Batches of tokens on the matrix cores (the shared expert of a chunk):
 // y[t][o] = sum over groups g of scale[o][g] * sum_{i in g} W[o][i] x[t][i],
 // as mvq_rows_f32 (src/simd_avx512.c:20-88) per token. v_mfma_f32_16x16x32_f16
@@ -6162,19 +6226,44 @@ extern "C" int wk_set_slots(warp_slot *table, const warp_slot_upd *u, int n, int
 // (each thread a strided partial, then the waves, in order), so it is
 // deterministic; it differs from the reference's sequential sum by fp32
 // rounding only. One block per token.
-__global__ __launch_bounds__(256) void k_rmsnorm(const float *__restrict__ x, const float *__restrict__ w, int n,
-                                                 float eps, float *__restrict__ o) {
+__global__ __launch_bounds__(256) void k_rmsnorm(const float *x, const float *__restrict__ w, int n, float eps,
+                                                 float *o) {
     __shared__ float red[4];
     const float *xt = x + (size_t)blockIdx.x * n;
-    float s = 0.0f;
-    for (int i = threadIdx.x; i < n; i += 256) s = __fadd_rn(s, __fmul_rn(xt[i], xt[i]));
+    float *ot = o + (size_t)blockIdx.x * n;
+    // The loads of up to RN elements per thread are issued at once (clamped),
+    // x kept for the second pass where it all fits and w loaded before the
+    // sum is known: one load per loop step waited 14 times in turn at 3584
+    // (10.5 us; 4.6 now).
+    constexpr int RN = 16;
+    float xr[RN], wr[RN], s = 0.0f;
+    auto load = [&](const float *p, float *r, int i0) {
+#pragma unroll
+        for (int j = 0; j < RN; j++) r[j] = p[min(i0 + j * 256 + (int)threadIdx.x, n - 1)];
+    };
+    load(w, wr, 0);
+    for (int i0 = 0; i0 < n; i0 += RN * 256) {
+        load(xt, xr, i0);
+#pragma unroll
+        for (int j = 0; j < RN; j++)
+            if (i0 + j * 256 + (int)threadIdx.x < n) s = __fadd_rn(s, __fmul_rn(xr[j], xr[j]));
+    }
     s = wave_sum(s);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
     __syncthreads();
     s = __fadd_rn(__fadd_rn(red[0], red[1]), __fadd_rn(red[2], red[3]));
     const float r = __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(__fdiv_rn(s, (float)n), eps)));
-    float *ot = o + (size_t)blockIdx.x * n;
-    for (int i = threadIdx.x; i < n; i += 256) ot[i] = __fmul_rn(__fmul_rn(xt[i], r), w[i]);
+    for (int i0 = 0; i0 < n; i0 += RN * 256) {
+        if (n > RN * 256) {
+            load(xt, xr, i0);
+            load(w, wr, i0);
+        }
+#pragma unroll
+        for (int j = 0; j < RN; j++) {
+            const int i = i0 + j * 256 + (int)threadIdx.x;
+            if (i < n) ot[i] = __fmul_rn(__fmul_rn(xr[j], r), wr[j]);
+        }
+    }
 }
 
 extern "C" int wk_rmsnorm(const float *x, const float *w, int T, int n, float eps, float *o, void *stream) {

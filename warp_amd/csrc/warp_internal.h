@@ -150,6 +150,10 @@ typedef struct {
 /* Whether the fused kernels take this shape: bits 8 or 4, 16-byte rows,
  * a group a multiple of one 16-byte chunk's weights, rows short enough. */
 int wk_shared_fast_ok(int H, const warp_shared_args *sa);
+/* h [T][inter] of T tokens x [T][H] in one launch, where wk_shared_h_ok
+ * (that shape, x 16-byte aligned and one row of it within 64 KiB). */
+int wk_shared_h_ok(const float *x, int H, const warp_shared_args *sa);
+int wk_shared_h(const float *x, int T, int H, const warp_shared_args *sa, int n_cu, void *stream);
 /* Router logits [E] of one token (the fast fixed-order tree) and, in the
  * same launch, the shared expert's h. */
 int wk_router_shared(const float *W, const float *x, int E, int H, float *logits, const warp_shared_args *sa,
