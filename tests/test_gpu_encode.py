@@ -17,7 +17,7 @@ import os
 import numpy as np
 import pytest
 
-from gpu_util import log
+from gpu_util import dev, empty, log
 from oracle import pyoracle as po
 
 pytestmark = pytest.mark.gpu
@@ -122,3 +122,95 @@ def test_encode_scores_never_decide(S, E, n):
         got, ref = wh.vq_encode(X, b), np.empty((n, S), np.uint16)
         po.lib().or_vq_encode(X.ctypes.data, n, b.ctypes.data, S, E, 8, ref.ctypes.data)
         assert np.array_equal(got, ref), (kind, int(np.count_nonzero(got != ref)))
+
+
+def spread_books(kind, rng, S, E):
+    """Codebooks whose entries differ in length, offset or not at all."""
+    b = rng.normal(0.0, 1.0, size=(S, E, 8)).astype(np.float32)
+    if kind == "one x100":
+        b[:, E // 2] *= np.float32(100.0)
+    elif kind == "three far":
+        b[:, E // 4] *= np.float32(1e4)
+        b[:, E // 2] *= np.float32(1e20)
+        b[:, E - 1, 3] = np.inf
+    elif kind == "heavy":
+        b /= np.sqrt(rng.chisquare(2, size=b.shape) / 2).astype(np.float32)
+    elif kind == "offset":
+        b[0] += np.float32(64.0)
+    elif kind == "copies":
+        b[:, E // 2:] = b[:, :E - E // 2]
+    elif kind == "near copies":
+        b[:, E // 2:] = b[:, :E - E // 2] * np.float32(1.0 + 2.0 ** -22)
+    elif kind == "zeros":
+        b[:, ::2] *= np.float32(0.0)                  # 0 and -0
+    return b
+
+
+SPREADS = ["one x100", "three far", "heavy", "offset", "copies", "near copies", "zeros"]
+
+
+@pytest.mark.parametrize("S,E,n", [(3, 256, 5000), (2, 33, 4999), (17, 33, 130), (2, 1500, 3000)])
+def test_encode_spread_codebooks(S, E, n):
+    """Codes of codebooks with a few long entries, heavy tails, an offset,
+    entries twice and almost twice, zeros of both signs: the oracle's. The
+    vectors are of the entries' kind, some of them entries."""
+    import warp_amd.hip as wh
+    for kind in SPREADS:
+        rng = np.random.default_rng(S * E + n)
+        b = spread_books(kind, rng, S, E)
+        X = spread_books(kind, rng, 1, n)[0]
+        X[::7] = b[0, rng.integers(0, E, len(X[::7]))]
+        X[~np.isfinite(X)] = 0.0
+        got, ref = wh.vq_encode(X, b), np.empty((n, S), np.uint16)
+        po.lib().or_vq_encode(X.ctypes.data, n, b.ctypes.data, S, E, 8, ref.ctypes.data)
+        assert np.array_equal(got, ref), (kind, int(np.count_nonzero(got != ref)))
+
+
+def test_encode_several_tiles_per_wave():
+    """Enough vectors that a wave takes several 64-vector tiles, the last ones
+    ragged: codes equal the oracle's, also where a tile's scan has the wave
+    scan the next ones too."""
+    import warp_amd.hip as wh
+    S, E, n = 2, 34, 2 * 262144 + 65
+    for kind in ("heavy", "near copies"):
+        rng = np.random.default_rng(5)
+        b = spread_books(kind, rng, S, E)
+        X = rng.normal(0.0, 1.0, size=(n, 8)).astype(np.float32)
+        got, ref = wh.vq_encode(X, b), np.empty((n, S), np.uint16)
+        po.lib().or_vq_encode(X.ctypes.data, n, b.ctypes.data, S, E, 8, ref.ctypes.data)
+        assert np.array_equal(got, ref), (kind, int(np.count_nonzero(got != ref)))
+
+
+def encode_ms(X, books, reps=20):
+    """The device's time of one warp_hip_vq_encode_dev of X [n][8]."""
+    import warp_amd.hip as wh
+    from warp_amd.device import Event
+    n, (S, E, _) = X.shape[0], books.shape
+    x, b, r, codes = dev(X), dev(books), empty((n, 8)), empty((n, S), np.uint16)
+
+    def go():
+        assert wh.lib().warp_hip_vq_encode_dev(x.ptr, n, b.ptr, S, E, r.ptr, codes.ptr, None) == 0
+    go()
+    best = np.inf
+    for _ in range(3):
+        e0, e1 = Event(), Event()
+        e0.record(None)
+        for _ in range(reps):
+            go()
+        e1.record(None)
+        e1.synchronize()
+        best = min(best, e0.elapsed_ms(e1) / reps)
+    return best
+
+
+def test_encode_time_hardly_depends_on_the_entries():
+    """A codebook with a long entry, heavy tails, an offset or copies takes no
+    more than 3 times the time of one without (measured: 2 at most, with
+    copies). Scanning every vector takes 4 times, one by one 8 times."""
+    rng = np.random.default_rng(9)
+    S, E, n = 3, 256, 400000
+    plain = encode_ms(rng.normal(size=(n, 8)).astype(np.float32), spread_books("", rng, S, E))
+    for kind in ("one x100", "heavy", "offset", "copies", "zeros"):
+        ms = encode_ms(spread_books(kind, rng, 1, n)[0], spread_books(kind, rng, S, E))
+        log(f"vq_encode {kind}: {ms * 1e3:.1f} us, {ms / plain:.2f} times the plain codebook's")
+        assert ms <= 3.0 * plain, (kind, ms, plain)

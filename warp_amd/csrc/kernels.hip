@@ -5717,34 +5717,42 @@ extern "C" int wk_combine_chunk(const float *y, const int *tok_slots, const floa
 // the scan was bound by them. Here the matrix cores find the winner and the
 // reference's arithmetic only confirms it. d / 2 orders entries as the score
 // |e|^2 / 2 - v . e + B does (B of the vector alone, about |v|^2 / 2), and one
-// v_mfma_f32_16x16x32_f16 gives 16 entries x 16 vectors of that: v and e,
-// scaled by a power of two that puts the codebook's largest component into
-// [512, 1024), are split into fp16 high and low parts, and the 32 products of
-// a pair are
+// v_mfma_f32_16x16x32_f16 gives 16 entries x 16 vectors of that: v and e, both
+// less a point amid the entries and scaled by a power of two (enc_scale), are
+// split into fp16 high and low parts, and the 32 products of a pair are
 //   k  0.. 7  -v high . e high      k 24..26  256 . (|e|^2 / 512 in three parts)
 //   k  8..15  -v high . e low       k 27      2^15 . (0, or past the codebook's
-//   k 16..23  -v low . e high                 end a value no score reaches)
+//   k 16..23  -v low . e high                 end, for an entry as long as
+//                                             ENC_FAR and for a copy of an
+//                                             earlier one a value no score
+//                                             reaches)
 //                                   k 28      B / 2^14 . 2^14
 // Scores are positive (B has a margin), so they compare as whole numbers. A
 // lane holds 4 entries of one vector; their least score, its low four bits
 // replaced by the number of the 16-entry tile, goes into a running least and
 // second least. So a wave has, for its 64 vectors, the best group
-// of 4 entries and a bound on every other group. If the second least is
-// further off than the scores can be wrong (see enc_margin), the reference's
-// winner is in that group, and its 4 entries are compared with the
-// reference's own arithmetic; any other vector (near ties, infinities, NaN,
-// magnitudes out of range) is scanned in full by the whole wave. Codes are
-// those of the scan in every case.
+// of 4 entries and a bound on every other group. The group's 4 entries are
+// compared with the reference's own arithmetic; if no other entry can be as
+// near as the nearest of them (enc_certain), that is the reference's winner.
+// Any other vector (near ties, infinities, NaN, magnitudes out of range) is
+// scanned: a few of a wave's one by one, each by the whole wave; more than
+// ENC_SERIAL all at once, a lane each, and the wave's next tiles then too,
+// without scores. Codes are those of the scan in every case.
 //
 // Bound by the vector instructions of the running minimum and the matrix
 // cores about alike. Stages whose codebooks fit LDS together go in one
 // launch, the residual in registers: 1,835,008 vectors, 3 x 256 entries,
-// 154 us (the scan: 698). A larger codebook goes one stage a launch, 1,024
-// entries staged at a time: the same vectors against 2 x 4,096, 1,519 us (the
-// scan: 7,674).
-constexpr int ENC_TILES = 96;                        // 16-entry tiles in LDS at most (1 KiB each), all stages in a launch
+// 138 us (the scan: 610 to 650). A larger codebook goes one stage a launch,
+// 1,024 entries staged at a time: 180,001 vectors against 2 x 4,096, 173 us
+// (the scan: 1,093). The same vectors with what codebooks hold besides: one
+// entry 100 times as long 145 and 201 us, tails of Student's t(2) 148 and 202,
+// entries and vectors 64 standard deviations from 0 the times above, every
+// entry twice 254 and 333.
+constexpr int ENC_TILES = 96;                        // 16-entry tiles in LDS at most (1 KiB each), of all stages
 constexpr int ENC_PIECE = 64;                        // tiles staged at a time when a stage's are more
 constexpr int ENC_STAGES = 16;                       // stages in a launch at most
+constexpr float ENC_FAR = 5400.0f;                   // an entry this long (scaled) has no score
+constexpr int ENC_SERIAL = 16;                       // vectors of a wave scanned one by one at most
 
 struct EncArgs {
     const float *src;                                // [n][8]
@@ -5755,17 +5763,26 @@ struct EncArgs {
     uint16_t *codes;                                 // [n][stages]
 };
 
-// How far below the least score of the other groups the winner's must be.
-// With V = |v|, E = max |e| (both scaled), the products of a score sum to at
-// most 1.01 (V + E)^2 / 2 + 2^15 in magnitude. A score's error is at most
-// 2^-17 of that (32 products added in fp32 in any order, truncated at worst:
-// 2^-18; the tile number in the four low bits: 2^-19; the products of the
-// splits' remainders: 2^-20) plus 2^-12 (V + E + 64) where parts fall below
-// the normal fp16 range; the reference's d / 2 is rounded by at most
-// 2^-20 (V + E)^2. Twice their sum, as two scores are compared.
-__device__ __forceinline__ float enc_margin(float V, float E) {
-    const float s = V + E;
-    return 2.02f * (0x1.4p-18f * s * s + 0x1p-12f * (s + 64.0f) + 0.25f);
+// Whether every entry outside the vector's best group is further off than the
+// group's nearest, at distance d / 2 = D (d as the reference computes it, D
+// scaled). k2 is the least score of those entries, but for its last four
+// bits; V = |v|, V2 its square, Bq the constant in the scores, E the longest
+// entry, infinite where an entry was taken for ENC_FAR.
+// An entry longer than R = V + sqrt(2 D) is further off than D whatever its
+// score says, so only entries within r = min(E, R) can be wrong by the error
+// of their scores: 2^-18 of the products' magnitudes (32 products added in
+// fp32 in any order, truncated at worst), which sum to 1.001 (V + r)^2 / 2 + Bq
+// - V^2 / 2; 2^-22 (V + r)^2 for the splits' remainders and the squares' sum;
+// 2^-24 (V + r)^2 for the rounding of v and e less the middle; 2^-12 (V + r + 80)
+// where fp16 parts fall below the normal range (taken as lost). k2's last bits
+// are 2^-19 of it, the reference's d is rounded by 2^-20 of it, and V2 and this
+// sum by 2^-21. (One entry 100 times the others, with E in the place of r and
+// the longest component setting the scale: nine vectors in ten were scanned.)
+__device__ __forceinline__ bool enc_certain(float k2, float V, float V2, float Bq, float E, float D) {
+    const float R = 1.001f * (V + __builtin_amdgcn_sqrtf(2.0f * D)), r = V + fminf(E, R);
+    const float err = 0x1.4p-18f * (0.5f * r * r + (Bq - 0.5f * V2)) + 0x1p-12f * (r + 80.0f) +
+                      0x1.4p-19f * (k2 + D) + 0x1p-20f * V2;
+    return (k2 - Bq) + 0.5f * V2 - D > err && V <= 16384.0f && (E < INFINITY || R <= ENC_FAR);
 }
 
 // the reference's distance
@@ -5804,53 +5821,155 @@ __device__ __forceinline__ EncBest enc_fold(const EncBest &x, const EncBest &y) 
     return enc_min(p, q);
 }
 
+// A point amid the entries: per component the median of three of them (0
+// where that is not finite). Scores of v and e less the same point order the
+// entries as those of v and e do, and stay accurate where an offset is large
+// beside the entries' differences.
+__device__ __forceinline__ void enc_mid(const f4 *b, int entries, float (&mid)[8]) {
+    const int c1 = entries >> 1, c2 = entries - 1;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const float m =
+            __builtin_amdgcn_fmed3f(b[j >> 2][j & 3], b[2 * c1 + (j >> 2)][j & 3], b[2 * c2 + (j >> 2)][j & 3]);
+        mid[j] = fabsf(m) < INFINITY ? m : 0.0f;
+    }
+}
+
+// A stage's scale: the largest component into [512, 1024), but the mean
+// exponent of the entries' largest components no lower than about 2^3, or a
+// few long entries would leave the others too few bits. most: the bits of the
+// largest component; exps: 2^19 times the number of entries with a finite one
+// other than 0, plus the sum of half their exponents. 1 where there is none
+// to take a scale from; 0 where that is out of range: such a codebook is
+// scanned.
+__device__ __forceinline__ float enc_scale(unsigned most, unsigned exps) {
+    const float mean = 2.0f * (float)(exps & 0x7ffffu) * __builtin_amdgcn_rcpf((float)(exps >> 19));
+    // the largest component is in [2^(e - 1), 2^e)
+    const int e = min((int)(most >> 23), (int)mean + 7) - 126;
+    return !exps ? 1.0f : e >= -40 && e <= 40 ? __uint_as_float((unsigned)(137 - e) << 23) : 0.0f;
+}
+
+// op over the wave's lanes, in every lane
+template <class Op> __device__ __forceinline__ unsigned enc_wave(unsigned x, Op op) {
+    const auto h = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    x = op(h[0], h[1]);
+    const auto q = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    x = op(q[0], q[1]);
+    x = op(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xf, 0xf, false));      // rotations of 16 lanes
+    x = op(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x124, 0xf, 0xf, false));
+    x = op(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x122, 0xf, 0xf, false));
+    return op(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x121, 0xf, 0xf, false));
+}
+
+// The reference's scan, a vector per lane: every lane meets the same entry at
+// once, so the entries come by scalar loads.
+__device__ __forceinline__ void enc_scan(const float *book, int entries, const float *v, int &best, float &bestd) {
+    typedef const __attribute__((address_space(4))) f4 cf4;
+    cf4 *b = (cf4 *)book;
+    best = 0;
+    bestd = INFINITY;
+#pragma unroll 4
+    for (int c = 0; c < entries; c++) {
+        const f4 e0 = b[2 * c], e1 = b[2 * c + 1];
+        const float d = enc_dist(v, make_float4(e0[0], e0[1], e0[2], e0[3]), make_float4(e1[0], e1[1], e1[2], e1[3]));
+        if (d < bestd) {
+            bestd = d;
+            best = c;
+        }
+    }
+}
+
 // PIECES: the launch's one stage is staged ENC_PIECE tiles at a time;
 // otherwise every stage's tiles are staged once and a block's waves go over
 // their 64-vector tiles on their own.
 template <bool PIECES>
 __global__ __launch_bounds__(1024) void k_vq_encode(EncArgs a) {
     extern __shared__ half8 enc_lds[];               // [tiles][64] operands, then [wave][3][64] vector operands
-    __shared__ unsigned s_max[ENC_STAGES], s_norm[ENC_STAGES];   // bits of max |component|, of max |e'|^2
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nt = (a.entries + 15) >> 4;
-    const int nw = blockDim.x >> 6;
-    half8 *xch = enc_lds + (PIECES ? ENC_PIECE : a.nst * nt) * 64 + wave * 192;
-    if (tid < ENC_STAGES) s_max[tid] = s_norm[tid] = 0u;
+    // per stage: bits of the largest |component|; the entries' number and the
+    // sum of their exponents (enc_scale); bits of the largest |e'|^2; the scale
+    // (0: not in range) and the middle
+    __shared__ unsigned s_max[ENC_STAGES], s_exp[ENC_STAGES], s_norm[ENC_STAGES];
+    __shared__ float s_scale[ENC_STAGES];
+    __shared__ __attribute__((aligned(16))) float s_mid[ENC_STAGES][8];
+    const int tid = threadIdx.x, lane = tid & 63, nt = (a.entries + 15) >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = blockDim.x >> 6;
+    half8 *xch = enc_lds + (PIECES ? ENC_PIECE : a.nst * nt) * 64;
+    // A hash table of the entries in LDS that is not in use yet: a slot keeps
+    // the first entry (of the first stage) that falls into it.
+    unsigned *tab = (unsigned *)(PIECES ? enc_lds : xch);
+    const unsigned nslot = PIECES ? ENC_PIECE * 256 : nw * 768;
+    __shared__ uint64_t s_dup[PIECES ? 64 : 1];      // entries equal to an earlier one
+    if (tid < ENC_STAGES) s_max[tid] = s_exp[tid] = s_norm[tid] = 0u;
+    for (int i = tid; i < (int)nslot; i += blockDim.x) tab[i] = ~0u;
     __syncthreads();
-    for (int s = 0; s < a.nst; s++) {
-        const uint4 *b = (const uint4 *)(a.books + (size_t)s * a.entries * 8);
+    auto slot_of = [&](int s, f4 e0, f4 e1) {
+        unsigned h = (unsigned)s;
+#pragma unroll
+        for (int j = 0; j < 8; j++)                   // (-0 as 0)
+            h = (h ^ __float_as_uint((j < 4 ? e0[j & 3] : e1[j & 3]) + 0.0f)) * 0x9E3779B1u;
+        return __umulhi(h, nslot);
+    };
+    // Whether an earlier entry is equal. Such an entry never wins, and without
+    // a score it ties with none. (One whose slot another entry has is not
+    // found: its vectors are scanned.)
+    auto is_dup = [&](int s, int c, f4 e0, f4 e1) {
+        const unsigned f = tab[slot_of(s, e0, e1)];
+        if (c >= a.entries || (int)(f >> 12) != s || (int)(f & 4095u) == c) return false;
+        const f4 *b = (const f4 *)(a.books + ((size_t)s * a.entries + (f & 4095u)) * 8);
+        const f4 x = b[0], y = b[1];
+        return x[0] == e0[0] && x[1] == e0[1] && x[2] == e0[2] && x[3] == e0[3] && y[0] == e1[0] && y[1] == e1[1] &&
+               y[2] == e1[2] && y[3] == e1[3];
+    };
+    const int nb = (a.entries + 63) >> 6;            // a wave takes 64 entries of a stage at a time
+    for (int it = wave; it < a.nst * nb; it += nw) {
+        const int s = it / nb, c = (it % nb) * 64 + lane;
+        const f4 *b = (const f4 *)(a.books + (size_t)s * a.entries * 8);
+        const f4 e0 = b[2 * min(c, a.entries - 1)], e1 = b[2 * min(c, a.entries - 1) + 1];
+        float mid[8];
+        enc_mid(b, a.entries, mid);
         unsigned m = 0;
-        for (int i = tid; i < a.entries * 2; i += blockDim.x) {
-            const uint4 w = b[i];
-            m = max(max(m, w.x & 0x7fffffffu), max(w.y & 0x7fffffffu, max(w.z & 0x7fffffffu, w.w & 0x7fffffffu)));
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            m = max(m, __float_as_uint((j < 4 ? e0[j & 3] : e1[j & 3]) - mid[j]) & 0x7fffffffu);
+        // (neither zero nor infinite nor NaN)
+        const bool in = c < a.entries && m - 1u < 0x7f7fffffu;
+        const unsigned most = enc_wave(in ? m : 0u, [](unsigned x, unsigned y) { return max(x, y); });
+        const unsigned ex = enc_wave(in ? 1u << 19 | m >> 24 : 0u, [](unsigned x, unsigned y) { return x + y; });
+        if (lane == 0) {
+            atomicMax(&s_max[s], most);
+            atomicAdd(&s_exp[s], ex);
         }
-        atomicMax(&s_max[s], m);                     // infinities and NaN come out largest
+        if (c < a.entries) atomicMin(&tab[slot_of(s, e0, e1)], (unsigned)(s << 12 | c));
+        if (c < 64 && lane < 8) s_mid[s][lane] = mid[lane];
     }
     __syncthreads();
-    // 2^x of a stage's scale; a codebook out of range is scanned in full
-    auto scale_of = [&](int s, bool &ok) {
-        const int e = (int)(s_max[s] >> 23) - 126;   // the largest component is in [2^(e - 1), 2^e)
-        ok = e >= -40 && e <= 40;
-        return ok ? ldexpf(1.0f, 10 - e) : 1.0f;
-    };
-    auto stage_tiles = [&](int s, int t0, int t1, half8 *to) {
-        bool ok;
-        const float sc = scale_of(s, ok);
-        const float *b = a.books + (size_t)s * a.entries * 8;
-        float most = 0.0f;
-        for (int c = t0 * 16 + tid; c < t1 * 16; c += blockDim.x) {
+    // tiles t0 .. t1 - 1 (t0 a multiple of 4) of stages s0 .. s1 - 1
+    auto stage_tiles = [&](int s0, int s1, int t0, int t1, half8 *to) {
+        const int nq = (t1 - t0 + 3) >> 2;
+        for (int it = wave; it < (s1 - s0) * nq; it += nw) {
+            const int s = s0 + it / nq, c = (t0 + (it % nq) * 4) * 16 + lane;
+            const float sc = enc_scale(s_max[s], s_exp[s]);
+            const f4 *b = (const f4 *)(a.books + (size_t)s * a.entries * 8);
+            const f4 e0 = b[2 * min(c, a.entries - 1)], e1 = b[2 * min(c, a.entries - 1) + 1];
+            const f4 m0 = *(const f4 *)s_mid[s], m1 = *(const f4 *)(s_mid[s] + 4);
             half8 h = {}, l = {}, k = {};
-            if (c < a.entries) {
-                const float4 e0 = ((const float4 *)b)[2 * c], e1 = ((const float4 *)b)[2 * c + 1];
-                const float e[8] = { e0.x, e0.y, e0.z, e0.w, e1.x, e1.y, e1.z, e1.w };
-                float nn = 0.0f;
+            float nn = 0.0f;
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const float x = e[j] * sc;
-                    h[j] = (_Float16)x;
-                    l[j] = (_Float16)(x - (float)h[j]);
-                    nn += x * x;
-                }
-                most = fmaxf(most, nn);
+            for (int j = 0; j < 8; j++) {
+                const float x = (j < 4 ? e0[j & 3] - m0[j & 3] : e1[j & 3] - m1[j & 3]) * sc;
+                h[j] = (_Float16)x;
+                l[j] = (_Float16)(x - (float)h[j]);
+                nn += x * x;
+            }
+            const bool dup = PIECES ? s_dup[c >> 6] >> lane & 1 : is_dup(s, c, e0, e1);
+            const bool in = c < a.entries && !dup, near = nn < ENC_FAR * ENC_FAR;       // (not NaN)
+            const unsigned most = enc_wave(!in ? 0u : near ? __float_as_uint(nn) : 0x7f800000u,
+                                           [](unsigned x, unsigned y) { return max(x, y); });
+            if (lane == 0) {
+                atomicMax(&s_norm[s], most);
+                s_scale[s] = sc;
+            }
+            if (in && near) {
                 nn *= 1.0f / 512.0f;
                 k[0] = (_Float16)nn;
                 nn -= (float)k[0];
@@ -5858,23 +5977,34 @@ __global__ __launch_bounds__(1024) void k_vq_encode(EncArgs a) {
                 nn -= (float)k[1];
                 k[2] = (_Float16)nn;
             } else {
+                h = l = half8{};
                 k[3] = (_Float16)60000.0f;
             }
             k[4] = (_Float16)16384.0f;
-            half8 *d = to + (size_t)((c >> 4) - t0) * 64 + (c & 15);
-            d[0] = h;
-            d[16] = l;
-            d[32] = h;
-            d[48] = k;
+            if (c < t1 * 16) {
+                half8 *d = to + (size_t)((s - s0) * (t1 - t0) + (c >> 4) - t0) * 64 + (c & 15);
+                d[0] = h;
+                d[16] = l;
+                d[32] = h;
+                d[48] = k;
+            }
         }
-        atomicMax(&s_norm[s], __float_as_uint(most));
     };
-    if (!PIECES) {
-        for (int s = 0; s < a.nst; s++) stage_tiles(s, 0, nt, enc_lds + (size_t)s * nt * 64);
+    if (PIECES) {
+        for (int it = wave; it < nb; it += nw) {
+            const int c = it * 64 + lane;
+            const f4 *b = (const f4 *)a.books;
+            const uint64_t dup = __ballot(is_dup(0, c, b[2 * min(c, a.entries - 1)], b[2 * min(c, a.entries - 1) + 1]));
+            if (lane == 0) s_dup[it] = dup;
+        }
+    } else {
+        stage_tiles(0, a.nst, 0, nt, enc_lds);
         __syncthreads();
     }
+    xch += wave * 192;
     const int kg = lane >> 4, col = lane & 15;
     const long ntile = (a.n + 63) >> 6, step = (long)gridDim.x * nw;
+    unsigned hard = 0, round = 0;                    // stages whose next tiles are scanned without scores
     // (PIECES: one tile per wave, and every wave takes part in the staging)
     for (long tile = (long)blockIdx.x * nw + wave; PIECES || tile < ntile; tile += step) {
         const long i = tile * 64 + lane;
@@ -5882,123 +6012,137 @@ __global__ __launch_bounds__(1024) void k_vq_encode(EncArgs a) {
         const float4 *src = (const float4 *)(a.src + (valid ? i : a.n - 1) * 8);
         const float4 v0 = src[0], v1 = src[1];
         float v[8] = { v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w };
+        if ((++round & 7) == 0) hard = 0;
         for (int s = 0; s < a.nst; s++) {
-            bool ok;
-            const float sc = scale_of(s, ok);
-            float V2 = 0.0f;
-            half8 h, l;
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const float x = -v[j] * sc;
-                h[j] = (_Float16)x;
-                l[j] = (_Float16)(x - (float)h[j]);
-                V2 += x * x;
-            }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            xch[lane] = h;
-            xch[64 + lane] = l;
-            // B: no score is negative, as E < 2900; rounded up (to at least 2)
-            const float V = sqrtf(V2), B = 0.5f * V2 + enc_margin(V, 2900.0f);
-            const half8 konst = { (_Float16)256.0f, (_Float16)256.0f, (_Float16)256.0f, (_Float16)32768.0f,
-                                  (_Float16)(B * 0x1.01p-14f + 0x1p-13f), (_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f };
-            xch[128 + lane] = konst;
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            half8 b[4];
-#pragma unroll
-            for (int q = 0; q < 4; q++) b[q] = xch[(kg == 3 ? 128 : kg == 2 ? 64 : 0) + q * 16 + col];
-            EncBest r[4];
-#pragma unroll
-            for (int q = 0; q < 4; q++) r[q] = { ~0u, ~0u, 0u };
-            // tiles t0 .. t1 - 1 of the stage, 16 (one tile number's worth) at a time
-            auto scan = [&](const half8 *fr, int t0, int t1) {
-                for (int c0 = t0; c0 < t1; c0 += 16, fr += 16 * 64) {
-                    unsigned c1[4], c2[4];
-#pragma unroll
-                    for (int q = 0; q < 4; q++) c1[q] = c2[q] = 0x7f800000u;
-                    auto tile16 = [&](int t) {
-                        const half8 av = fr[t * 64 + lane];
-                        f4 d[4];
-#pragma unroll
-                        for (int q = 0; q < 4; q++)
-                            d[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, b[q], f4{ 0.0f, 0.0f, 0.0f, 0.0f }, 0, 0, 0);
-#pragma unroll
-                        for (int q = 0; q < 4; q++) {
-                            unsigned g = min(min(__float_as_uint(d[q][0]), __float_as_uint(d[q][1])),
-                                             min(__float_as_uint(d[q][2]), __float_as_uint(d[q][3])));
-                            g = (g & ~15u) | (unsigned)t;
-                            // the median: c1 <= c2, all positive
-                            c2[q] = __float_as_uint(__builtin_amdgcn_fmed3f(__uint_as_float(c1[q]), __uint_as_float(c2[q]),
-                                                                            __uint_as_float(g)));
-                            c1[q] = min(c1[q], g);
-                        }
-                    };
-                    const int nc = min(16, t1 - c0);
-                    int t = 0;
-                    for (; t + 4 <= nc; t += 4) {
-                        tile16(t);
-                        tile16(t + 1);
-                        tile16(t + 2);
-                        tile16(t + 3);
-                    }
-                    for (; t < nc; t++) tile16(t);
-#pragma unroll
-                    for (int q = 0; q < 4; q++)
-                        r[q] = enc_min(r[q], { c1[q], c2[q], (unsigned)(c0 * 4) + (c1[q] & 15u) * 4 + kg });
-                }
-            };
-            if (PIECES) {
-                for (int t0 = 0; t0 < nt; t0 += ENC_PIECE) {
-                    const int t1 = min(t0 + ENC_PIECE, nt);
-                    __syncthreads();                 // the piece before is done with
-                    stage_tiles(s, t0, t1, enc_lds);
-                    __syncthreads();
-                    scan(enc_lds, t0, t1);
-                }
-            } else {
-                scan(enc_lds + (size_t)s * nt * 64, 0, nt);
-            }
-            // lane l gets vector l's: tiles 0 and 2, 1 and 3 by halves, then by rows
-            const EncBest w = enc_fold<16>(enc_fold<32>(r[0], r[2]), enc_fold<32>(r[1], r[3]));
-            const float E = sqrtf(__uint_as_float(s_norm[s]));
-            const bool cert = ok && V <= 16384.0f && __uint_as_float(w.k2) - __uint_as_float(w.k1) > enc_margin(V, E);
-            const float4 *bk = (const float4 *)(a.books + (size_t)s * a.entries * 8);
+            const float *book = a.books + (size_t)s * a.entries * 8;
+            const float4 *bk = (const float4 *)book;
+            const float sc = PIECES ? enc_scale(s_max[s], s_exp[s]) : s_scale[s];
+            bool cert = false;
             int best = 0;
             float bestd = INFINITY;
+            if (sc > 0.0f && !(hard >> s & 1)) {     // (uniform; with PIECES in the block)
+                const f4 m0 = *(const f4 *)s_mid[s], m1 = *(const f4 *)(s_mid[s] + 4);
+                float V2 = 0.0f;
+                half8 h, l;
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int c = (int)w.id * 4 + u, cc = min(c, a.entries - 1);
-                const float d = enc_dist(v, bk[2 * cc], bk[2 * cc + 1]);
-                if (c < a.entries && d < bestd) {
-                    bestd = d;
-                    best = c;
+                for (int j = 0; j < 8; j++) {
+                    const float x = ((j < 4 ? m0[j & 3] : m1[j & 3]) - v[j]) * sc;
+                    h[j] = (_Float16)x;
+                    l[j] = (_Float16)(x - (float)h[j]);
+                    V2 += x * x;
                 }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                xch[lane] = h;
+                xch[64 + lane] = l;
+                // B, above |v|^2 / 2 by more than a score near 0 can be wrong: by
+                // 0.003 of it and 1.9
+                const _Float16 bq = (_Float16)(0.5f * V2 * 0x1.01p-14f + 0x1p-13f);
+                const half8 konst = { (_Float16)256.0f, (_Float16)256.0f, (_Float16)256.0f, (_Float16)32768.0f,
+                                      bq, (_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f };
+                xch[128 + lane] = konst;
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                half8 b[4];
+#pragma unroll
+                for (int q = 0; q < 4; q++) b[q] = xch[(kg == 3 ? 128 : kg == 2 ? 64 : 0) + q * 16 + col];
+                EncBest r[4];
+#pragma unroll
+                for (int q = 0; q < 4; q++) r[q] = { ~0u, ~0u, 0u };
+                // tiles t0 .. t1 - 1 of the stage, 16 (one tile number's worth) at a time
+                auto scan = [&](const half8 *fr, int t0, int t1) {
+                    for (int c0 = t0; c0 < t1; c0 += 16, fr += 16 * 64) {
+                        unsigned c1[4], c2[4];
+#pragma unroll
+                        for (int q = 0; q < 4; q++) c1[q] = c2[q] = 0x7f800000u;
+                        auto tile16 = [&](int t) {
+                            const half8 av = fr[t * 64 + lane];
+                            f4 d[4];
+#pragma unroll
+                            for (int q = 0; q < 4; q++)
+                                d[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, b[q], f4{}, 0, 0, 0);
+#pragma unroll
+                            for (int q = 0; q < 4; q++) {
+                                unsigned g = min(min(__float_as_uint(d[q][0]), __float_as_uint(d[q][1])),
+                                                 min(__float_as_uint(d[q][2]), __float_as_uint(d[q][3])));
+                                g = (g & ~15u) | (unsigned)t;
+                                // the median: c1 <= c2, all positive
+                                c2[q] = __float_as_uint(__builtin_amdgcn_fmed3f(
+                                    __uint_as_float(c1[q]), __uint_as_float(c2[q]), __uint_as_float(g)));
+                                c1[q] = min(c1[q], g);
+                            }
+                        };
+                        const int nc = min(16, t1 - c0);
+                        int t = 0;
+                        for (; t + 4 <= nc; t += 4) {
+                            tile16(t);
+                            tile16(t + 1);
+                            tile16(t + 2);
+                            tile16(t + 3);
+                        }
+                        for (; t < nc; t++) tile16(t);
+#pragma unroll
+                        for (int q = 0; q < 4; q++)
+                            r[q] = enc_min(r[q], { c1[q], c2[q], (unsigned)(c0 * 4) + (c1[q] & 15u) * 4 + kg });
+                    }
+                };
+                if (PIECES) {
+                    for (int t0 = 0; t0 < nt; t0 += ENC_PIECE) {
+                        const int t1 = min(t0 + ENC_PIECE, nt);
+                        __syncthreads();                 // the piece before is done with
+                        stage_tiles(s, s + 1, t0, t1, enc_lds);
+                        __syncthreads();
+                        scan(enc_lds, t0, t1);
+                    }
+                } else {
+                    scan(enc_lds + (size_t)s * nt * 64, 0, nt);
+                }
+                // lane l gets vector l's: tiles 0 and 2, 1 and 3 by halves, then by rows
+                const EncBest w = enc_fold<16>(enc_fold<32>(r[0], r[2]), enc_fold<32>(r[1], r[3]));
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const int c = (int)w.id * 4 + u, cc = min(c, a.entries - 1);
+                    const float d = enc_dist(v, bk[2 * cc], bk[2 * cc + 1]);
+                    if (c < a.entries && d < bestd) {
+                        bestd = d;
+                        best = c;
+                    }
+                }
+                cert = enc_certain(__uint_as_float(w.k2), __builtin_amdgcn_sqrtf(V2), V2, (float)bq * 16384.0f,
+                                   __builtin_amdgcn_sqrtf(__uint_as_float(s_norm[s])), 0.5f * bestd * sc * sc);
             }
-            for (uint64_t todo = __ballot(valid && !cert); todo; todo &= todo - 1) {
-                const int at = __ffsll((unsigned long long)todo) - 1;
-                float x[8];
+            const uint64_t open = __ballot(valid && !cert);
+            if (__popcll(open) > ENC_SERIAL) {
+                enc_scan(book, a.entries, v, best, bestd);
+                hard |= 1u << s;
+            } else {
+                for (uint64_t todo = open; todo; todo &= todo - 1) {
+                    const int at = __ffsll((unsigned long long)todo) - 1;
+                    float x[8];
 #pragma unroll
-                for (int j = 0; j < 8; j++) x[j] = __shfl(v[j], at);
-                float md = INFINITY;
-                int mc = 0x7fffffff;
-                for (int c = lane; c < a.entries; c += 64) {
-                    const float d = enc_dist(x, bk[2 * c], bk[2 * c + 1]);
-                    if (d < md) {
-                        md = d;
-                        mc = c;
+                    for (int j = 0; j < 8; j++) x[j] = __shfl(v[j], at);
+                    float md = INFINITY;
+                    int mc = 0x7fffffff;
+#pragma unroll 4
+                    for (int c0 = 0; c0 < a.entries; c0 += 64) {
+                        const int c = min(c0 + lane, a.entries - 1);
+                        const float d = enc_dist(x, bk[2 * c], bk[2 * c + 1]);
+                        if (d < md) {
+                            md = d;
+                            mc = c;
+                        }
                     }
-                }
 #pragma unroll
-                for (int o = 32; o > 0; o >>= 1) {
-                    const float od = __shfl_xor(md, o);
-                    const int oc = __shfl_xor(mc, o);
-                    if (od < md || (od == md && oc < mc)) {
-                        md = od;
-                        mc = oc;
+                    for (int o = 32; o > 0; o >>= 1) {
+                        const float od = __shfl_xor(md, o);
+                        const int oc = __shfl_xor(mc, o);
+                        if (od < md || (od == md && oc < mc)) {
+                            md = od;
+                            mc = oc;
+                        }
                     }
+                    if (lane == at) best = md < INFINITY ? mc : 0;
                 }
-                if (lane == at) best = md < INFINITY ? mc : 0;
             }
             if (valid) a.codes[i * a.stages + a.stage0 + s] = (uint16_t)best;
             if (a.stage0 + s + 1 < a.stages) {

@@ -124,9 +124,10 @@ int wk_router_cert(const float *W, const float *x, int E, int H, const float *bi
 int wk_mvq(const int8_t *W, const uint16_t *ws, size_t rowbytes, int group, int bits,
            const float *x, int M, int N, int T, float *y, void *stream);
 
-/* The encoder (waste_vq_encode for 8-dim vectors): one launch per stage; codes
- * [n][stages] 16-bit; cur [n][8] holds the residual between stages (unused
- * for one stage). X, books and cur 16-byte aligned; entries <= 4096. */
+/* The encoder (waste_vq_encode for 8-dim vectors): stages whose codebooks fit
+ * LDS together in one launch; codes [n][stages] 16-bit; cur [n][8] holds the
+ * residual between launches (unused for one stage). X, books and cur 16-byte
+ * aligned; entries <= 4096. */
 int wk_vq_encode(const float *X, long n, const float *books, int stages, int entries, float *cur,
                  uint16_t *codes, void *stream);
 /* One Lloyd iteration (waste_vq_lloyd) on device buffers: assignment into asg,
