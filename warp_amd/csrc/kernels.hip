@@ -2947,24 +2947,31 @@ static int launch_vq_t(const VqArgs &a, int nkinds, int max_units, int npg, int 
 // 384 experts of 2 x 4096 at 7168 x 2048: 1,026 -> 911 and 580 -> 474 us, LDS
 // active 93% of the time, two thirds of that in conflicts.
 //
-// A run kernel's codebooks in LDS. 4096 entries a stage: as they are. 256
-// entries: stages 0 and 1 in 16 copies each, the third stage (what is left of
-// the 160 KiB) in 8, where two lanes still share a column half the time.
-// at[s]: the lane's base for stage s.
-template <int FMT> struct RunBooks {
+// A run kernel's codebooks in LDS. 4096 entries a stage: as they are, at
+// addresses without a lane's part. 256 entries: stages 0 and 1 in 16 copies
+// each, the third stage (what is left of the 160 KiB) in 8, where two lanes
+// still share a column half the time. ONE: the copies of stages 0 and 1 of an
+// entry follow each other, so that one register holds the lane's part of both
+// addresses: the reduced-precision kernel has none to spare (with a register
+// per stage it kept 16 others in memory at three stages, with this 3, none of
+// them in its loop: 512 tokens through 64 experts at 2304 x 1024 262 -> 250
+// us). The exact kernel has them, and is 1% slower so.
+template <int FMT, bool ONE> struct RunBooks {
     typedef FmtT<FMT> F;
     static constexpr bool REP = F::E == 256;
     static constexpr int VECS = REP ? 256 * (F::S == 3 ? 40 : 32) : F::S * F::E;   // 16-byte vectors
-    const unsigned char *at[F::S];
+    // stages 0 and 1: bytes from an entry to the next, and from stage to stage
+    static constexpr unsigned STEP = ONE ? 512 : 256, STAGE = ONE ? 256 : 65536;
+    const unsigned char *lds;
+    unsigned at[F::S];
     static __device__ __forceinline__ void stage(uint4 *dst, const uint16_t *books) {
         const uint4 *src = (const uint4 *)books;
         for (int i = threadIdx.x; i < VECS; i += blockDim.x)
-            dst[i] = src[!REP ? i : i < 8192 ? i >> 4 : 512 + ((i - 8192) >> 3)];
+            dst[i] = src[!REP ? i : i >= 8192 ? 512 + ((i - 8192) >> 3) : ONE ? (i >> 4 & 1) * 256 + (i >> 5) : i >> 4];
     }
-    __device__ __forceinline__ RunBooks(const uint4 *lds, int lane) {
+    __device__ __forceinline__ RunBooks(const uint4 *to, int lane) : lds((const unsigned char *)to) {
 #pragma unroll
-        for (int s = 0; s < F::S; s++)
-            at[s] = (const unsigned char *)lds + (!REP ? s * 65536 : s * 65536 + 16 * (lane & (s < 2 ? 15 : 7)));
+        for (int s = 0; s < F::S; s++) at[s] = s < 2 ? 16 * (lane & 15) + s * STAGE : 131072 + 16 * (lane & 7);
     }
     // the vectors of 4 consecutive rows at one position
     __device__ __forceinline__ void gather(const Word<F::SB> &wd, half8 (&a)[4][F::S]) const {
@@ -2973,8 +2980,8 @@ template <int FMT> struct RunBooks {
             const unsigned sl = wd.slot(t);
 #pragma unroll
             for (int s = 0; s < F::S; s++) {
-                const unsigned c = REP ? (sl >> (8 * s)) & 0xFFu : s ? sl >> 12 : sl & 0xFFFu;
-                a[t][s] = *(const half8 *)(at[s] + c * (!REP ? 16u : s < 2 ? 256u : 128u));
+                const unsigned c = (sl >> (8 * s)) & 0xFFu;
+                a[t][s] = *(const half8 *)(lds + (!REP ? cb_off<FMT>(sl, s) : c * (s < 2 ? STEP : 128u) + at[s]));
             }
         }
     }
@@ -2983,7 +2990,7 @@ template <int FMT> struct RunBooks {
 // one unit: the rows of block rb of the NT jobs from j0
 template <int FMT, int WD, int NT>
 __device__ __forceinline__ void run_unit(const VqArgs &a, const warp_job *jobs, float *y, int j0, int rb, int lane,
-                                         const RunBooks<FMT> &cb) {
+                                         const RunBooks<FMT, false> &cb) {
     typedef FmtT<FMT> F;
     const int M = a.M, nv = a.N >> 3, npg = nv >> 2;
     const int g = lane >> 4, jc = lane & 15, ts = jc >> 1, hl = jc & 1;
@@ -3094,7 +3101,7 @@ __device__ __forceinline__ void run_unit(const VqArgs &a, const warp_job *jobs, 
 template <int FMT, int WD1, int WD2>
 __global__ __launch_bounds__(1024) void k_vq_mfma_run(VqArgs a, const int *__restrict__ runs) {
     typedef FmtT<FMT> F;
-    __shared__ uint4 cb_lds[RunBooks<FMT>::VECS];
+    __shared__ uint4 cb_lds[RunBooks<FMT, false>::VECS];
     const int kind = a.kind_lo + blockIdx.y;
     const warp_job *jobs = a.jobs + (size_t)kind * a.max_jobs;
     const int nrb = (a.M + 63) >> 6;
@@ -3103,11 +3110,11 @@ __global__ __launch_bounds__(1024) void k_vq_mfma_run(VqArgs a, const int *__res
         rq_leave(rq, threadIdx.x, rq.nw);
         return;
     }
-    RunBooks<FMT>::stage(cb_lds, a.books + (size_t)kind * F::S * F::E * 8);
+    RunBooks<FMT, false>::stage(cb_lds, a.books + (size_t)kind * F::S * F::E * 8);
     __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (wave >= rq.nw) return;
-    const RunBooks<FMT> cb(cb_lds, lane);
+    const RunBooks<FMT, false> cb(cb_lds, lane);
     for (int l = rq_first(rq) + wave; l < rq.n;) {
         const int u = rq_unit(rq, l);
         const int rv = __builtin_amdgcn_readfirstlane(runs[u / nrb]);   // uniform: u is
@@ -3159,7 +3166,7 @@ template <int FMT, int WD>
 __global__ __launch_bounds__(1024) void k_vq_run_f16(VqArgs a, const int *__restrict__ runs) {
     typedef FmtT<FMT> F;
     constexpr int NWB = 16, RB = WARP_RUN_J / 2;            // waves per block; B operands (2 jobs each) per step
-    __shared__ uint4 cb_lds[RunBooks<FMT>::VECS];
+    __shared__ uint4 cb_lds[RunBooks<FMT, true>::VECS];
     const int kind = a.kind_lo + blockIdx.y;
     const warp_job *jobs = a.jobs + (size_t)kind * a.max_jobs;
     const int M = a.M, N = a.N, nv = N >> 3, npg = nv >> 2, nrb = (M + 63) >> 6;
@@ -3168,11 +3175,13 @@ __global__ __launch_bounds__(1024) void k_vq_run_f16(VqArgs a, const int *__rest
         rq_leave(rq, threadIdx.x, rq.nw);
         return;
     }
-    RunBooks<FMT>::stage(cb_lds, a.books + (size_t)kind * F::S * F::E * 8);
+    RunBooks<FMT, true>::stage(cb_lds, a.books + (size_t)kind * F::S * F::E * 8);
     __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    // (uniform: the queue's divisions on scalar registers)
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     if (wave >= rq.nw) return;
-    const RunBooks<FMT> cb(cb_lds, lane);
+    const RunBooks<FMT, true> cb(cb_lds, lane);
     const int g = lane >> 4, jc = lane & 15;
     // B and the code words through buffer loads: a per-lane offset fixed for
     // the unit and a per-group offset in a scalar register
