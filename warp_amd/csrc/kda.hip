@@ -57,7 +57,9 @@ __global__ __launch_bounds__(KDA_NT) void k_kda(int T, int H, int K, int V, int 
                                                 float *__restrict__ S, float *__restrict__ o) {
     constexpr int RS = 16 * R, LS = RS + 4;       // rows per column; LDS stride (steps on different banks)
     constexpr int TT = R == 16 ? 16 : 32, NE = TT * RS / KDA_NT;
-    __shared__ float dk[TT * LS], kv[TT * LS], qv[TT * LS], vt[TT * 16], bt[TT], nrm[2 * TT];
+    __shared__ __attribute__((aligned(16))) float kv[TT * LS], qv[TT * LS];
+    __shared__ float dk[TT * LS], vt[TT * 16], bt[TT], nrm[2 * TT];
+    static_assert(LS % 4 == 0 && __alignof__(kv) >= 16 && __alignof__(qv) >= 16, "their rows are read as float4");
     // blocks reach the XCDs in turn: each takes a contiguous eighth of the
     // units, so a head's blocks share one L2
     const int per = (int)gridDim.x >> 3, unit = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);

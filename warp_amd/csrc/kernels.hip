@@ -1241,7 +1241,7 @@ __global__ __launch_bounds__(256) void k_router_shared(const float *__restrict__
         if (threadIdx.x == 0) logits[blockIdx.x] = v;
         return;
     }
-    extern __shared__ float xl[];
+    extern __shared__ __attribute__((aligned(16))) float xl[];
     using Q = QRow<BITS, MC>;
     const int r = ((int)blockIdx.x - E) * 4 + (int)(threadIdx.x >> 6), rr = min(r, sa.inter - 1);
     const int nc = H / Q::WPC, ng = H / sa.group;
@@ -5116,7 +5116,8 @@ __global__ __launch_bounds__(1024) void k_lut_p6(const float *__restrict__ x, co
                                                  float lbeta, int8_t *__restrict__ lut8,
                                                  float *__restrict__ lscale) {
     __shared__ float xsh[WARP_LUT_BLK * 8];
-    __shared__ int8_t out[WARP_LUT_BLK * 256];
+    __shared__ __attribute__((aligned(16))) int8_t out[WARP_LUT_BLK * 256];
+    static_assert(__alignof__(out) >= 16, "read as uint4");
     const int vec = blockIdx.y, blk = blockIdx.x, nv = N >> 3, nblk = (nv + WARP_LUT_BLK - 1) / WARP_LUT_BLK;
     const int tid = threadIdx.x, e = tid & 255, g = tid >> 8;
     const int v0 = blk * WARP_LUT_BLK, nvb = min(WARP_LUT_BLK, nv - v0);
