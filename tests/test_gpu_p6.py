@@ -43,6 +43,41 @@ def test_matvec_bits(hidden, inter):
         ctx.close()
 
 
+@pytest.mark.parametrize("shift", [1, 2, 3])
+def test_matvec_index_blocks_at_any_byte(shift):
+    """A record's header may put its index blocks at any byte; the code words
+    are read four bytes at a time."""
+    import warp_amd
+    hidden, inter = 328, 200
+    model = model_of(hidden, inter)
+    ctx = open_ctx(model)
+    try:
+        warp_amd.load_container_model(ctx, model)
+        bT = po.books_T(model.books_raw)
+        raw = model.layers[0].records[5]
+        r, hdr = np.frombuffer(raw, np.uint8), np.frombuffer(raw[:48], np.uint32)
+        off = [int(v) for v in hdr[5:9]]
+        rows = 2 * (2 * inter + hidden)
+        moved, at = np.zeros_like(r), []
+        for k, (a, e) in enumerate(zip(off, off[1:] + [off[3] + rows])):
+            at.append(a + (4 * k + 4 + shift if k < 3 else 16))
+            moved[at[k]:at[k] + e - a] = r[a:e]
+        moved[:48] = r[:48]
+        moved[20:36] = np.array(at, np.uint32).view(np.uint8)
+        rec = dev(moved)
+        rng = np.random.default_rng(shift)
+        for kind in range(3):
+            M, N = (inter, hidden) if kind < 2 else (hidden, inter)
+            x, y = rng.normal(size=N).astype(np.float32), empty(M)
+            ctx.vq_matvec(0, kind, rec, dev(x), y)
+            s0 = off[3] + 2 * (0, inter, 2 * inter)[kind]
+            ref = po.vq_matvec("VQ4P", r[off[kind]:].copy(), r[s0:s0 + 2 * M].view(np.uint16).copy(), x, bT, kind * 4,
+                               M, N)
+            assert np.array_equal(host(y), ref), kind
+    finally:
+        ctx.close()
+
+
 @pytest.mark.parametrize("hidden,inter,experts,T", [(328, 200, 6, 1), (328, 200, 6, 5), (328, 200, 6, 23),
                                                     (264, 520, 40, 150), (2080, 136, 6, 37)])
 def test_chunk_jobs(hidden, inter, experts, T):

@@ -2594,6 +2594,7 @@ template <> struct FmtT<WARP_FMT_VQ12> { static constexpr int S = 2, E = 4096, S
 // Device memory seen as global (not generic) memory, so that loads through
 // pointers read from job lists are global loads.
 typedef const __attribute__((address_space(1))) unsigned gu32;
+typedef const __attribute__((address_space(1), aligned(1))) unsigned gu32b;      // starting at any byte
 
 // Code word of 4 consecutive rows at one position, as loaded by a lane.
 template <int SB> struct Word;
@@ -2605,6 +2606,10 @@ template <> struct Word<3> {
     }
     __device__ __forceinline__ void load_keep(const uint8_t *p) {
         const gu32 *q = (const gu32 *)p;
+        w = u3v{q[0], q[1], q[2]};
+    }
+    __device__ __forceinline__ void load_any(const uint8_t *p) {
+        const gu32b *q = (const gu32b *)p;
         w = u3v{q[0], q[1], q[2]};
     }
     __device__ __forceinline__ void mask(unsigned m) { w = u3v{w.x & m, w.y & m, w.z & m}; }
@@ -5216,7 +5221,8 @@ __device__ __forceinline__ void p6_rows(const P6Args &a, const warp_job &jb, int
         Word<3> wd[D];
         const int k0 = p0 / 4 + sub * GP;
         auto word = [&](int j, int k) {
-            wd[j].load_keep(idx + (size_t)min((k0 + min(k, GP - 1)) * 4 + g, nv - 1) * 192);
+            // (an index block starts at the byte that the record's header says)
+            wd[j].load_any(idx + (size_t)min((k0 + min(k, GP - 1)) * 4 + g, nv - 1) * 192);
         };
 #pragma unroll
         for (int j = 0; j < D; j++) word(j, j);
