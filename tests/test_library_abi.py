@@ -55,3 +55,24 @@ def test_open_refuses_without_a_device():
     with pytest.raises(warp_amd.WarpHipError):
         warp_amd.Context(hidden=128, inter=64, n_experts=8, top_k=2, n_layers=1, fmt="VQ3R",
                          rec_bytes=12288, cache_bytes=12288 * 8)
+
+
+def test_run_kernels_refuse_longer_runs_than_they_take():
+    """A run list made for the reduced-precision kernel holds runs of four
+    jobs; the exact one would leave out two of them."""
+    import warp_amd
+    from warp_amd.device import device_count
+    if device_count() > 0:
+        pytest.skip("a device is present: the calls that are not refused would launch")
+    L, buf = warp_amd.lib(), (ctypes.c_char * 4096)()
+    at = (ctypes.addressof(buf) + 15) & ~15
+    y = (ctypes.c_void_p * 3)(at, at, at)
+    L.wk_vq_runs.argtypes = [ctypes.c_int] + [ctypes.c_void_p] * 2 + [ctypes.c_int, ctypes.c_void_p] + [
+        ctypes.c_int] * 2 + [ctypes.c_void_p] * 4 + [ctypes.c_int] * 4 + [ctypes.c_void_p, ctypes.c_int,
+                                                                         ctypes.c_void_p]
+
+    def call(fp16_rows, run_j):
+        return L.wk_vq_runs(9, at, at, 1, at, 0, 1, at, at, at, y, 64, 32, fp16_rows, run_j, at, 256, None)
+    for fp16_rows, most in ((0, 2), (8, 4)):
+        assert call(fp16_rows, most) < -1000              # passed the checks: no device to launch on
+        assert [call(fp16_rows, r) for r in (0, most + 1, 5)] == [-1] * 3

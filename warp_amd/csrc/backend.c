@@ -2157,10 +2157,11 @@ static int chunk_experts(warp_hip_ctx *c, int layer, const layer_t *B, const flo
     const warp_hip_cfg *g = &c->cfg;
     const int E = g->n_experts, K = g->top_k, H = c->He, I = g->inter, P = T * K; /* H: the experts' width */
     const warp_slot *table = c->table_dev + (size_t)layer * E;
+    const int run_j = prefill_fp16(c) ? WARP_RUN_J : WARP_RUN_JX;
     KRN(c, wait_copies(c));
     KRN(c, wk_plan_chunk(c->idx, c->w, T, K, E, table, c->counts, c->offsets, c->pair_tok, c->pair_exp, c->pair_w,
                          c->tok_slots, c->jobs, c->max_jobs, c->njobs, c->runs, c->missing, I, e_lo, e_hi, !first,
-                         prefill_fp16(c) ? WARP_RUN_J : WARP_RUN_JX, c->st));
+                         run_j, c->st));
     DEV(c, hipEventRecord(c->ev_before, c->st));
     float *yk[3] = { c->yg, c->yu, c->yd };
     if (c->P6) {
@@ -2184,19 +2185,19 @@ static int chunk_experts(warp_hip_ctx *c, int layer, const layer_t *B, const flo
                 KRN(c, wk_split_pgm(X_dev, NULL, c->pair_tok, c->offsets + E, P, H, 0, 0, 0.0f, 0.0f, c->xsp,
                                     c->xscalep, c->st));
             KRN(c, wk_vq_runs(g->fmt, c->jobs, c->njobs, c->max_jobs, c->runs, 0, 2, B->books, c->xsp, c->xscalep,
-                              yk, I, H, P, c->run_queue, c->st));
+                              yk, I, H, P, run_j, c->run_queue, c->n_cu, c->st));
             KRN(c, wk_split_pgm(c->yg, c->yu, NULL, c->offsets + E, P, I, 1, g->act_situ, g->situ_beta,
                                 g->situ_linear_beta, c->xsh, c->xscaleh, c->st));
             KRN(c, wk_vq_runs(g->fmt, c->jobs, c->njobs, c->max_jobs, c->runs, 2, 1, B->books, c->xsh, c->xscaleh,
-                              yk, H, I, P, c->run_queue, c->st));
+                              yk, H, I, P, run_j, c->run_queue, c->n_cu, c->st));
         } else {
             if (first) KRN(c, wk_split(X_dev, T, H, c->xs, c->xscale, c->st));
             KRN(c, wk_vq_runs(g->fmt, c->jobs, c->njobs, c->max_jobs, c->runs, 0, 2, B->books, c->xs, c->xscale, yk,
-                              I, H, 0, c->run_queue, c->st));
+                              I, H, 0, run_j, c->run_queue, c->n_cu, c->st));
             KRN(c, wk_act_split(c->yg, c->yu, P, I, g->act_situ, g->situ_beta, g->situ_linear_beta, c->xsh,
                                 c->xscaleh, NULL, c->st));
             KRN(c, wk_vq_runs(g->fmt, c->jobs, c->njobs, c->max_jobs, c->runs, 2, 1, B->books, c->xsh, c->xscaleh,
-                              yk, H, I, 0, c->run_queue, c->st));
+                              yk, H, I, 0, run_j, c->run_queue, c->n_cu, c->st));
         }
     }
     return 0;

@@ -3132,11 +3132,11 @@ __global__ __launch_bounds__(1024) void k_vq_mfma_run(VqArgs a, const int *__res
 }
 
 template <int FMT>
-static int launch_vq_run(const VqArgs &a, const int *runs, int nkinds, int max_units, void *stream) {
+static int launch_vq_run(const VqArgs &a, const int *runs, int nkinds, int max_units, int n_cu, void *stream) {
     typedef FmtT<FMT> F;
     constexpr int WD1 = F::S == 3 ? 4 : 6, WD2 = F::S == 3 ? 2 : 3;
     // one block per CU: the kinds of a launch share the CUs
-    int grid = 256 / nkinds;
+    int grid = max(n_cu / nkinds, 1);
     if (grid > max_units) grid = max_units;
     grid = (grid + RQ_GROUPS - 1) / RQ_GROUPS * RQ_GROUPS;   // the unit queues' groups
     hipLaunchKernelGGL((k_vq_mfma_run<FMT, WD1, WD2>), dim3(grid, nkinds), dim3(1024), 0, (hipStream_t)stream, a, runs);
@@ -3318,10 +3318,10 @@ __global__ __launch_bounds__(1024) void k_vq_run_f16(VqArgs a, const int *__rest
 }
 
 template <int FMT>
-static int launch_vq_run_f16(const VqArgs &a, const int *runs, int nkinds, int max_units, void *stream) {
+static int launch_vq_run_f16(const VqArgs &a, const int *runs, int nkinds, int max_units, int n_cu, void *stream) {
     typedef FmtT<FMT> F;
     constexpr int WD = F::S == 3 ? 2 : 3;                   // code words and B operands in flight
-    int grid = 256 / nkinds;                                // one block per CU: the kinds share the CUs
+    int grid = max(n_cu / nkinds, 1);                       // one block per CU: the kinds share the CUs
     if (grid > max_units) grid = max_units;
     grid = (grid + RQ_GROUPS - 1) / RQ_GROUPS * RQ_GROUPS;   // the unit queues' groups
     hipLaunchKernelGGL((k_vq_run_f16<FMT, WD>), dim3(grid, nkinds), dim3(1024), 0, (hipStream_t)stream, a, runs);
@@ -3331,9 +3331,11 @@ static int launch_vq_run_f16(const VqArgs &a, const int *runs, int nkinds, int m
 
 extern "C" int wk_vq_runs(int fmt, const warp_job *jobs, const int *njobs, int max_jobs, const int *runs,
                           int kind_lo, int nkinds, const uint16_t *books, const uint16_t *xs, const float *xscale,
-                          float *const *y, int M, int N, int fp16_rows, unsigned *queue, void *stream) {
+                          float *const *y, int M, int N, int fp16_rows, int run_j, unsigned *queue, int n_cu,
+                          void *stream) {
     if (M <= 0 || N <= 0 || (N % 32) || max_jobs <= 0 || !runs || !queue || kind_lo < 0 || nkinds < 1 || kind_lo + nkinds > 3 ||
-        fp16_rows < 0 || (size_t)fp16_rows * N * 2 >= ((size_t)1 << 31))
+        fp16_rows < 0 || (size_t)fp16_rows * N * 2 >= ((size_t)1 << 31) || run_j < 1 ||
+        run_j > (fp16_rows ? WARP_RUN_J : WARP_RUN_JX) || n_cu < 1)
         return -1;
     for (int k = kind_lo; k < kind_lo + nkinds; k++)
         if ((uintptr_t)y[k] & 15) return -1;                // (16-byte row stores)
@@ -3354,8 +3356,8 @@ extern "C" int wk_vq_runs(int fmt, const warp_job *jobs, const int *njobs, int m
     const int max_units = max_jobs * ((M + 63) / 64);
     switch (fmt) {
 #define VR(F)                                                                                                      \
-    return fp16 ? launch_vq_run_f16<F>(a, runs, nkinds, max_units, stream)                                         \
-                : launch_vq_run<F>(a, runs, nkinds, max_units, stream)
+    return fp16 ? launch_vq_run_f16<F>(a, runs, nkinds, max_units, n_cu, stream)                                   \
+                : launch_vq_run<F>(a, runs, nkinds, max_units, n_cu, stream)
     case WARP_FMT_VQ3R: VR(WARP_FMT_VQ3R);
     case WARP_FMT_VQ2R: VR(WARP_FMT_VQ2R);
     case WARP_FMT_VQ12: VR(WARP_FMT_VQ12);

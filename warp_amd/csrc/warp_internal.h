@@ -180,8 +180,9 @@ int wk_vq_matvec(int fmt, const warp_job *jobs, const int *njobs, int max_jobs,
                  const float *xscale, float *const *y, int M, int N, int tokens_per_job,
                  void *stream);
 /* The same for prefill by runs: runs[0..njobs[3]) = (first job << 3) | jobs,
- * up to WARP_RUN_J (exact products: WARP_RUN_JX) consecutive jobs of one
- * expert (wk_plan_chunk writes them); each run's records are decoded once for all its jobs.
+ * up to run_j consecutive jobs of one expert (the run_j that wk_plan_chunk
+ * wrote them with; -1 above WARP_RUN_J, for exact products WARP_RUN_JX);
+ * each run's records are decoded once for all its jobs.
  * fp16_rows = 0: exact products, xs/xscale as for wk_vq_matvec (rows by
  * xi). fp16_rows > 0: the reduced-precision products (stage vectors added
  * in fp16, x's fp16 high half), xs [N/32][fp16_rows][32] and xscale
@@ -192,7 +193,7 @@ int wk_vq_matvec(int fmt, const warp_job *jobs, const int *njobs, int max_jobs,
 #define WARP_RUNQ_WORDS 1536
 int wk_vq_runs(int fmt, const warp_job *jobs, const int *njobs, int max_jobs, const int *runs,
                int kind_lo, int nkinds, const uint16_t *books, const uint16_t *xs, const float *xscale,
-               float *const *y, int M, int N, int fp16_rows, unsigned *queue, void *stream);
+               float *const *y, int M, int N, int fp16_rows, int run_j, unsigned *queue, int n_cu, void *stream);
 /* Inputs of the reduced-precision products: rows p < *nrows of
  * act(g, u) (act = 1, pair rows; SiLU with the hardware exp, SiTU exact)
  * or of x row rowmap[p] (act = 0, u NULL),
