@@ -4,6 +4,8 @@ tables of several LDS passes, jobs of 1 to 8 tokens, and launches with one
 and with four row blocks per block. A matvec is bit for bit the oracle's
 (integer sums and a fixed order of fp32 folds); layers meet the 1e-4 bar.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -81,8 +83,7 @@ def test_matvec_index_blocks_at_any_byte(shift):
 @pytest.mark.parametrize("hidden,inter,experts,T", [(328, 200, 6, 1), (328, 200, 6, 5), (328, 200, 6, 23),
                                                     (264, 520, 40, 150), (2080, 136, 6, 37)])
 def test_chunk_jobs(hidden, inter, experts, T):
-    """T = 150 over 40 experts: 450 pairs on 2 x 9 row blocks take the launch
-    with four row blocks per block; the others the one with one."""
+    """Launches with one row block per block (few jobs, or few row blocks)."""
     import warp_amd
     model = model_of(hidden, inter, experts)
     ctx = open_ctx(model, max_tokens=T)
@@ -94,5 +95,34 @@ def test_chunk_jobs(hidden, inter, experts, T):
         ctx.sync()
         ref = po.LayerView(model, 0).moe_chunk(X)[0]
         assert rel_err(host(out), ref) <= 1e-4
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("hidden,inter,T", [(264, 712, 150), (264, 840, 150), (1416, 728, 151)])
+def test_chunk_four_row_blocks(hidden, inter, T):
+    """Launches with four row blocks per block: gate and up of 12 and of 14
+    row blocks (the last group partial), and at 1416 the down rows' 23 too.
+    The jobs hold 1, 2, 3 to 4 and 5 to 8 tokens, a kernel loop each."""
+    import warp_amd
+    from warp_amd.device import rt
+    experts, top_k = 40, 3
+    n = ctypes.c_int()
+    assert rt().hipDeviceGetAttribute(ctypes.byref(n), 63, 0) == 0 and n.value > 0     # multiprocessor count
+    n_cu = n.value
+    jobs = min(T * top_k, T * top_k // 8 + experts + 1)     # the most that a list holds
+    blocks = lambda M: (M + 63) // 64
+    assert jobs * 2 * blocks(inter) >= 8 * n_cu and (hidden < 1416 or jobs * blocks(hidden) >= 8 * n_cu)
+    model = model_of(hidden, inter, experts, top_k)
+    ctx = open_ctx(model, max_tokens=T)
+    try:
+        warp_amd.load_container_model(ctx, model)
+        X = np.random.default_rng(T).normal(size=(T, hidden)).astype(np.float32)
+        out, route, _ = ctx.moe_chunk_host(0, X)
+        counts = np.bincount(route.ravel(), minlength=experts)
+        sizes = set(int(n) for c in counts for n in [8] * (c // 8) + [c % 8])
+        assert {1, 2, 8} <= sizes and sizes & {3, 4}, sizes
+        ref = po.LayerView(model, 0).moe_chunk(X)[0]
+        assert rel_err(out, ref) <= 1e-4
     finally:
         ctx.close()
