@@ -1106,7 +1106,7 @@ def run_vq_encode(args):
         e1.record(None)
         e1.synchronize()
         ms = e0.elapsed_ms(e1) / args.steps
-        ops = n * S_ * E_ * 64.0                     # per entry: 32 products of the score
+        ops = n * S_ * E_ * 16.0                     # per entry: v . e, not the score's split parts
         res[f"{S_}x{E_}"] = {"ms_per_matrix": round(ms, 3), "vectors_per_s": round(n / (ms / 1e3), 1),
                              "mfma_flops": ops / (ms / 1e3), "mfma_frac": round(ops / (ms / 1e3) / F16_PEAK_FLOPS, 4)}
         log(f"bench: vq-encode {S_}x{E_}: {ms:.3f} ms per matrix")

@@ -197,6 +197,8 @@ __global__ __launch_bounds__(KDA_NT) void k_kda(int T, int H, int K, int V, int 
 extern "C" int wk_kda(int T, int H, int K, int V, const float *q, const float *k, const float *v, const float *g,
                       const float *beta, float *S, float *o, void *stream) {
     if (T <= 0 || H <= 0 || K <= 0 || K > KDA_MAX_K || V <= 0 || V > 1024) return -1;
+    // (the header's bound on K V, which callers test and fall back by; nothing
+    // here needs it since the state left LDS)
     if ((size_t)K * V * sizeof(float) > 150 * 1024) return -1;
     const int units = H * ((V + 15) / 16);
     const dim3 grid((unsigned)((units + 7) / 8 * 8));
