@@ -5904,23 +5904,23 @@ __device__ __forceinline__ void enc_scan(const float *book, int entries, const f
 // (8.3), 3 x 32 entries 15.0 (16.5); at 1,835,008 vectors 16.6 (26.4), 27.8
 // (31.2) and 75.6 (78.3). 48 entries: 7.6 (8.7), but 39.2 (33.1).
 __global__ __launch_bounds__(256) void k_vq_scan(EncArgs a) {
-    const long i = (long)blockIdx.x * 256 + threadIdx.x;
-    if (i >= a.n) return;
-    const float4 *src = (const float4 *)(a.src + i * 8);
-    const float4 v0 = src[0], v1 = src[1];
-    float v[8] = { v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w };
-    for (int s = 0; s < a.nst; s++) {
-        const float *book = a.books + (size_t)s * a.entries * 8;
-        int best;
-        float bestd;
-        enc_scan(book, a.entries, v, best, bestd);
-        a.codes[i * a.stages + s] = (uint16_t)best;
-        if (s + 1 < a.nst) {
-            const float4 *e = (const float4 *)book + 2 * best;
-            const float4 e0 = e[0], e1 = e[1];
-            const float x[8] = { e0.x, e0.y, e0.z, e0.w, e1.x, e1.y, e1.z, e1.w };
+    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < a.n; i += (long)gridDim.x * 256) {
+        const float4 *src = (const float4 *)(a.src + i * 8);
+        const float4 v0 = src[0], v1 = src[1];
+        float v[8] = { v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w };
+        for (int s = 0; s < a.nst; s++) {
+            const float *book = a.books + (size_t)s * a.entries * 8;
+            int best;
+            float bestd;
+            enc_scan(book, a.entries, v, best, bestd);
+            a.codes[i * a.stages + s] = (uint16_t)best;
+            if (s + 1 < a.nst) {
+                const float4 *e = (const float4 *)book + 2 * best;
+                const float4 e0 = e[0], e1 = e[1];
+                const float x[8] = { e0.x, e0.y, e0.z, e0.w, e1.x, e1.y, e1.z, e1.w };
 #pragma unroll
-            for (int j = 0; j < 8; j++) v[j] = __fsub_rn(v[j], x[j]);
+                for (int j = 0; j < 8; j++) v[j] = __fsub_rn(v[j], x[j]);
+            }
         }
     }
 }
@@ -6213,7 +6213,9 @@ extern "C" int wk_vq_encode(const float *X, long n, const float *books, int stag
     if (((uintptr_t)X | (uintptr_t)books | (uintptr_t)cur) & 15) return -1;
     if (entries <= ENC_SCAN) {
         EncArgs a = { X, nullptr, books, n, entries, stages, 0, stages, codes };
-        hipLaunchKernelGGL(k_vq_scan, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, a);
+        // (a launch holds fewer than 2^32 threads; more vectors take turns)
+        const unsigned grid = (unsigned)min((n + 255) / 256, 1L << 22);
+        hipLaunchKernelGGL(k_vq_scan, dim3(grid), dim3(256), 0, (hipStream_t)stream, a);
         CHECK_LAUNCH();
         return 0;
     }
