@@ -1124,7 +1124,7 @@ def run_vq_encode(args):
         "config": {"workload": "encode one K3 gate matrix (2048 x 7168 weights, 1,835,008 vectors of 8) with "
                                "3 x 256 codebooks (the reference's format); 2 x 4096 (16-bit codes) beside it",
                    "vectors": n, "parallelism": "single GPU"},
-        "passes": {k: {kk: (round(vv, 1) if isinstance(vv, float) and kk != "mfma_frac" else vv)
+        "passes": {k: {kk: (round(vv, 1) if kk in ("vectors_per_s", "mfma_flops") else vv)
                        for kk, vv in v.items()} for k, v in res.items()},
         "roofline": {"bound": "mfma", "achieved": round(main["mfma_flops"] / 1e12, 2),
                      "peak": round(F16_PEAK_FLOPS / 1e12, 2), "unit": "TFLOP/s fp16",

@@ -2950,7 +2950,7 @@ static int launch_vq_t(const VqArgs &a, int nkinds, int max_units, int npg, int 
 // for four jobs whatever the run had, one copy, before); 8 copies gave 204 and
 // 110, with LDS active 7.8 cycles per gather instead of 5.3. 32 tokens through
 // 384 experts of 2 x 4096 at 7168 x 2048: 1,026 -> 911 and 580 -> 474 us, LDS
-// active 93% of the time, two thirds of that in conflicts.
+// active in 97% of the CUs' busy cycles, two thirds of that in conflicts.
 //
 // A run kernel's codebooks in LDS. 4096 entries a stage: as they are, at
 // addresses without a lane's part. 256 entries: stages 0 and 1 in 16 copies
@@ -5757,15 +5757,16 @@ extern "C" int wk_combine_chunk(const float *y, const int *tok_slots, const floa
 // ENC_SERIAL all at once, a lane each, and the wave's next tiles then too,
 // without scores. Codes are those of the scan in every case.
 //
-// Bound by the vector instructions of the running minimum and the matrix
-// cores about alike. Stages whose codebooks fit LDS together go in one
-// launch, the residual in registers: 1,835,008 vectors, 3 x 256 entries,
-// 138 us (the scan: 610 to 650). A larger codebook goes one stage a launch,
-// 1,024 entries staged at a time: 180,001 vectors against 2 x 4,096, 173 us
-// (the scan: 1,093). The same vectors with what codebooks hold besides: one
-// entry 100 times as long 145 and 201 us, tails of Student's t(2) 148 and 202,
-// entries and vectors 64 standard deviations from 0 the times above, every
-// entry twice 254 and 333.
+// Bound by the running minimum's vector instructions and the matrix cores in
+// turn: 0.8 vector instructions a cycle and CU (a plain scan reaches 1.6), the
+// matrix cores busy 28% of the time, the waves waiting for a third of theirs.
+// Stages whose codebooks fit LDS together go in one launch, the residual in
+// registers: 1,835,008 vectors, 3 x 256 entries, 138 us (the scan: 610 to 650).
+// A larger codebook goes one stage a launch, 1,024 entries staged at a time:
+// 180,001 vectors against 2 x 4,096, 173 us (the scan: 1,093). The same vectors
+// with what codebooks hold besides: one entry 100 times as long 145 and 201 us,
+// tails of Student's t(2) 148 and 202, entries and vectors 64 standard
+// deviations from 0 the times above, every entry twice 254 and 333.
 constexpr int ENC_TILES = 96;                        // 16-entry tiles in LDS at most (1 KiB each), of all stages
 constexpr int ENC_PIECE = 64;                        // tiles staged at a time when a stage's are more
 constexpr int ENC_STAGES = 16;                       // stages in a launch at most
