@@ -89,6 +89,21 @@ def test_kda_tiles_and_remainders(T, H, K, V):
         assert np.array_equal(np.isnan(got), nan) and np.array_equal(bits(got)[~nan], bits(ref)[~nan])
 
 
+@pytest.mark.parametrize("K", [5, 24, 72, 96, 97, 160, 192])
+def test_kda_query_scale(K):
+    """1 / sqrt(K) where K is no square: a square root off by an ulp (the bare
+    hardware instruction's at 96) would show in every output."""
+    rng = np.random.default_rng(K)
+    T, H, V = 6, 3, 32
+    f32 = lambda a: np.ascontiguousarray(a, np.float32)
+    q, k = f32(rng.normal(size=(T, H, K))), f32(rng.normal(size=(T, H, K)))
+    v, gl = f32(rng.normal(size=(T, H, V))), f32(-rng.uniform(0, 3, size=(T, H, K)))
+    beta, S0 = f32(rng.uniform(0, 1, size=(T, H))), f32(rng.normal(size=(H, K, V)) * 0.1)
+    Sr, orf = po.kda_forward(q, k, v, gl, beta, S0)
+    S, o = forward_dev(q, k, v, gl, beta, S0)
+    assert np.array_equal(bits(S), bits(Sr)) and np.array_equal(bits(o), bits(orf))
+
+
 def test_kda_slot_through_the_table():
     import warp_amd
     calls = []
